@@ -45,7 +45,7 @@ struct alignas(64) QNode {
     uint8_t q[24];      // lo_x[4] hi_x[4] lo_y[4] hi_y[4] lo_z[4] hi_z[4]
     uint32_t child[4];  // as WideNode
     uint8_t count[4];   // as WideNode (at most kMaxLeafPrims)
-    uint32_t _pad1;
+    uint8_t tag[4];     // bits 27..31 of the child's stack entry: kLeafBit and count - 1 (0: internal, empty)
 };
 static_assert(sizeof(QNode) == 64, "QNode is 64 bytes");
 
@@ -133,6 +133,9 @@ __device__ inline float4 ldg_f4(const void* p) {
     const f32x4_t v = *(const __attribute__((address_space(1))) f32x4_t*)p;
     return make_float4(v.x, v.y, v.z, v.w);
 }
+__device__ inline double pair_f64(uint32_t lo, uint32_t hi) { return __hiloint2double(int(hi), int(lo)); }
+__device__ inline uint64_t pair_u64(uint32_t lo, uint32_t hi) { return uint64_t(hi) << 32 | lo; }
+__device__ inline float3 as_f3(uint4 w) { return make_float3(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z)); }
 __device__ inline uint32_t ldg_u32(const void* p) { return *(const __attribute__((address_space(1))) uint32_t*)p; }
 
 // ------------------------------------------------------------ float3 math

@@ -155,13 +155,14 @@ __device__ inline void quantize_axis(const float lo[4], const float hi[4], const
 __device__ inline QNode quantize_node(const WideNode& w) {
     QNode q;
     q._pad0 = 0;
-    q._pad1 = 0;
     quantize_axis(w.lo_x, w.hi_x, w.child, q.origin[0], q.exp[0], q.q + 0, q.q + 4);
     quantize_axis(w.lo_y, w.hi_y, w.child, q.origin[1], q.exp[1], q.q + 8, q.q + 12);
     quantize_axis(w.lo_z, w.hi_z, w.child, q.origin[2], q.exp[2], q.q + 16, q.q + 20);
     for (int k = 0; k < 4; k++) {
         q.child[k] = w.child[k];
         q.count[k] = uint8_t(w.count[k]);
+        // child | tag << 24 is the traversal's stack entry (a leaf's child is below 2^27)
+        q.tag[k] = w.count[k] ? uint8_t(0x80u | (w.count[k] - 1u) << 3) : uint8_t(0);
     }
     return q;
 }

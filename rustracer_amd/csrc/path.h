@@ -46,7 +46,7 @@ struct AlphaAnyHit {
     const SceneView* sv;
     const TlasView* tl;
     Rng4* rng;
-    __device__ bool ignore(uint32_t inst, uint32_t prim, float u, float v) {
+    __device__ __forceinline__ bool ignore(uint32_t inst, uint32_t prim, float u, float v) {
         return alpha_test_ignores(*sv, tl->inst[inst].custom_index, prim, u, v, *rng);
     }
 };

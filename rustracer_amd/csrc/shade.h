@@ -128,7 +128,7 @@ __device__ inline double bilerp(double t00, double t10, double t01, double t11, 
     return top + b * (bot - top);
 }
 
-__device__ inline D4 sample_texture(const SceneView& sv, int32_t index, double u, double v) {
+__device__ __forceinline__ D4 sample_texture(const SceneView& sv, int32_t index, double u, double v) {
     if (index < 0 || uint32_t(index) >= sv.num_textures) return D4{1.0, 1.0, 1.0, 1.0};
     const rt_texture& t = sv.textures[index];
     int W = int(t.width), H = int(t.height);
@@ -265,7 +265,7 @@ __device__ inline D4 sample_cube(const rt_texture& t, const float* lut, D3 d) {
 }
 
 // getUV, lib/RayTracingCommons.glsl:65-72
-__device__ inline D4 tex_uv(const SceneView& sv, rt_texture_info ti, D4 uv) {
+__device__ __forceinline__ D4 tex_uv(const SceneView& sv, rt_texture_info ti, D4 uv) {
     uint32_t c = uint32_t(ti.tex_coord);
     double u = 0, v = 0;
     if (c == 0u) { u = uv.x; v = uv.y; }
@@ -531,7 +531,7 @@ __device__ inline D3 offset_ray(D3 pd, D3 nd) {
 
 // ----------------------------------------------------------------- any-hit
 // RayTracing.rahit / RayTracing.shadow.rahit:44-104.  True = ignore the candidate.
-__device__ inline bool alpha_test_ignores(const SceneView& sv, uint32_t custom_index, uint32_t prim, float fu, float fv,
+__device__ __forceinline__ bool alpha_test_ignores(const SceneView& sv, uint32_t custom_index, uint32_t prim, float fu, float fv,
                                           Rng4& rng) {
     if (custom_index >= sv.num_prim_infos) return false;
     const rt_prim_info pi = sv.prim_infos[custom_index];
