@@ -277,9 +277,11 @@ struct Traversal {
             // order the hit children near-to-far: continue with the nearest, push the
             // others far first
 #define RT_CSWAP(i, j)                                                         \
-    if (key[j] < key[i]) {                                                     \
-        float tk = key[i]; key[i] = key[j]; key[j] = tk;                       \
-        uint32_t te = ent[i]; ent[i] = ent[j]; ent[j] = te;                    \
+    {                                                                          \
+        const bool s_ = key[j] < key[i];                                       \
+        const float tk = s_ ? key[j] : key[i], th = s_ ? key[i] : key[j];      \
+        const uint32_t te = s_ ? ent[j] : ent[i], tf = s_ ? ent[i] : ent[j];   \
+        key[i] = tk; key[j] = th; ent[i] = te; ent[j] = tf;                    \
     }
             RT_CSWAP(0, 1) RT_CSWAP(2, 3) RT_CSWAP(0, 2) RT_CSWAP(1, 3) RT_CSWAP(1, 2)
 #undef RT_CSWAP
