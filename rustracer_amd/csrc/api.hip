@@ -132,6 +132,7 @@ struct rt_ctx {
     bool mega_persistent = true;       // RT_OPTION_MEGAKERNEL_PERSISTENT
     uint32_t* d_next_pixel = nullptr;  // pixel counter of the persistent megakernel and adjoint
     uint32_t finish = 65536; // RT_OPTION_WAVEFRONT_FINISH
+    ScratchPool scratch;     // of the builds on this context's stream
     bool stage_timing = false;
     StageTimer timer;  // events of the last trace when stage_timing is set
 };
@@ -162,6 +163,13 @@ struct DeviceGuard {
     ~DeviceGuard() {
         if (prev >= 0) (void)hipSetDevice(prev);
     }
+};
+
+// One build's use of the context's scratch.
+struct ScratchScope {
+    ScratchPool& pool;
+    ScratchScope(ScratchPool& p, size_t bytes) : pool(p) { pool.begin(bytes); }
+    ~ScratchScope() { pool.end(); }
 };
 
 template <class T> T* dev_alloc(size_t count, hipError_t* e) {
@@ -414,30 +422,25 @@ int rt_build_blas_batch(rt_ctx* ctx, const rt_blas_input* inputs, uint32_t count
     const uint32_t n = uint32_t(total);
     hipStream_t st = ctx->stream;
     hipError_t e;
-    DevPtr d_segs(dev_alloc<TriSegment>(count, &e));
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-    DevPtr d_seg_start(dev_alloc<uint32_t>(count + 1, &e));
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-    DevPtr d_tri_in(dev_alloc<float4>(3 * size_t(n) + 3, &e));
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-    DevPtr d_lo(dev_alloc<float4>(n + 1, &e));
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-    DevPtr d_hi(dev_alloc<float4>(n + 1, &e));
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-    DevPtr d_bad(dev_alloc<uint32_t>(1, &e));
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-    RT_HIP(ctx, hipMemcpyAsync(d_segs.get(), segs.data(), sizeof(TriSegment) * count, hipMemcpyHostToDevice, st), "copy segments");
-    RT_HIP(ctx, hipMemcpyAsync(d_seg_start.get(), seg_start.data(), sizeof(uint32_t) * (count + 1), hipMemcpyHostToDevice, st), "copy segments");
-    RT_HIP(ctx, hipMemsetAsync(d_bad.get(), 0, sizeof(uint32_t), st), "memset");
-    int rc = prepare_triangles(st, (const TriSegment*)d_segs.get(), count, n, (float4*)d_tri_in.get(),
-                               (float4*)d_lo.get(), (float4*)d_hi.get(), (uint32_t*)d_bad.get());
+    ScratchScope scope(ctx->scratch, lbvh_scratch_bytes(n, count) + 80 * size_t(n) + (sizeof(TriSegment) + 4) * size_t(count));
+    ScratchPool& sc = ctx->scratch;
+    TriSegment* d_segs = sc.alloc<TriSegment>(count);
+    uint32_t* d_seg_start = sc.alloc<uint32_t>(count + 1);
+    float4* d_tri_in = sc.alloc<float4>(3 * size_t(n) + 3);
+    float4* d_lo = sc.alloc<float4>(n + 1);
+    float4* d_hi = sc.alloc<float4>(n + 1);
+    uint32_t* d_bad = sc.alloc<uint32_t>(1);
+    if (!d_segs || !d_seg_start || !d_tri_in || !d_lo || !d_hi || !d_bad)
+        return fail(ctx, RT_ERR_OUT_OF_MEMORY, "BLAS build: out of device memory");
+    RT_HIP(ctx, hipMemcpyAsync(d_segs, segs.data(), sizeof(TriSegment) * count, hipMemcpyHostToDevice, st), "copy segments");
+    RT_HIP(ctx, hipMemcpyAsync(d_seg_start, seg_start.data(), sizeof(uint32_t) * (count + 1), hipMemcpyHostToDevice, st), "copy segments");
+    RT_HIP(ctx, hipMemsetAsync(d_bad, 0, sizeof(uint32_t), st), "memset");
+    int rc = prepare_triangles(st, d_segs, count, n, d_tri_in, d_lo, d_hi, d_bad);
     if (rc) return hip_fail(ctx, hipError_t(rc), "prepare_triangles");
     LbvhResult res;
     std::string err;
-    rc = lbvh_build(st, (const float4*)d_lo.get(), (const float4*)d_hi.get(), n, (const uint32_t*)d_seg_start.get(),
-                    seg_start, ctx->leaf_max, ctx->collapse, ctx->treelets, &res, &err);
+    rc = lbvh_build(st, d_lo, d_hi, n, d_seg_start, seg_start, ctx->leaf_max, ctx->collapse, ctx->treelets, sc, &res, &err);
     if (rc) return fail(ctx, rc == int(hipErrorOutOfMemory) ? RT_ERR_OUT_OF_MEMORY : RT_ERR_HIP, "BLAS build: " + err);
-    DevPtr perm(res.perm), seg_bounds(res.seg_bounds);
     auto pool = std::make_shared<BlasPool>();
     pool->nodes.reset(res.nodes);
     pool->tris.reset(dev_alloc<float4>(3 * size_t(n) + 3, &e));
@@ -450,12 +453,12 @@ int rt_build_blas_batch(rt_ctx* ctx, const rt_blas_input* inputs, uint32_t count
     pool->num_tris = n;
     pool->level_start = res.level_start;
     for (uint32_t i = 0; i < count; i++) pool->prim_count.push_back(inputs[i].primitive_count);
-    rc = reorder_triangles(st, (const float4*)d_tri_in.get(), (const uint32_t*)perm.get(), n, (float4*)pool->tris.get());
+    rc = reorder_triangles(st, d_tri_in, res.perm, n, (float4*)pool->tris.get());
     if (rc) return hip_fail(ctx, hipError_t(rc), "reorder_triangles");
     std::vector<float> hb(6 * size_t(count));
     uint32_t bad = 0;
-    RT_HIP(ctx, hipMemcpyAsync(hb.data(), seg_bounds.get(), sizeof(float) * hb.size(), hipMemcpyDeviceToHost, st), "copy bounds");
-    RT_HIP(ctx, hipMemcpyAsync(&bad, d_bad.get(), sizeof(uint32_t), hipMemcpyDeviceToHost, st), "copy flag");
+    RT_HIP(ctx, hipMemcpyAsync(hb.data(), res.seg_bounds, sizeof(float) * hb.size(), hipMemcpyDeviceToHost, st), "copy bounds");
+    RT_HIP(ctx, hipMemcpyAsync(&bad, d_bad, sizeof(uint32_t), hipMemcpyDeviceToHost, st), "copy flag");
     RT_HIP(ctx, hipStreamSynchronize(st), "hipStreamSynchronize");
     if (bad) return fail(ctx, RT_ERR_INVALID_ARGUMENT, "an index exceeds max_vertex");
     std::vector<BlasDesc> descs(count);
@@ -649,25 +652,24 @@ int rt_build_tlas(rt_ctx* ctx, const rt_instance* d_instances, uint32_t count, r
     std::vector<InstanceRecord> trecs(nt);
     for (uint32_t k = 0; k < nt; k++) trecs[k] = recs[tlas_ids[k]];
     hipError_t e;
-    DevPtr d_rec(dev_alloc<InstanceRecord>(nt + 1, &e));
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-    DevPtr d_lo(dev_alloc<float4>(nt + 1, &e));
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-    DevPtr d_hi(dev_alloc<float4>(nt + 1, &e));
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
+    const uint32_t fn = uint32_t(flat_total);
+    ScratchScope scope(ctx->scratch, lbvh_scratch_bytes(nt, 1) + (sizeof(InstanceRecord) + 32) * size_t(nt) +
+                                         (fn ? lbvh_scratch_bytes(fn, 1) + 80 * size_t(fn) + sizeof(FlatSource) * nf : 0));
+    ScratchPool& sc = ctx->scratch;
+    InstanceRecord* d_rec = sc.alloc<InstanceRecord>(nt + 1);
+    float4* d_lo = sc.alloc<float4>(nt + 1);
+    float4* d_hi = sc.alloc<float4>(nt + 1);
+    uint32_t* d_seg = sc.alloc<uint32_t>(2);
+    if (!d_rec || !d_lo || !d_hi || !d_seg) return fail(ctx, RT_ERR_OUT_OF_MEMORY, "TLAS build: out of device memory");
     std::vector<uint32_t> seg_start = {0u, nt};
-    DevPtr d_seg(dev_alloc<uint32_t>(2, &e));
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-    if (nt) RT_HIP(ctx, hipMemcpyAsync(d_rec.get(), trecs.data(), sizeof(InstanceRecord) * nt, hipMemcpyHostToDevice, st), "copy records");
-    RT_HIP(ctx, hipMemcpyAsync(d_seg.get(), seg_start.data(), sizeof(uint32_t) * 2, hipMemcpyHostToDevice, st), "copy segments");
-    int rc = prepare_instances(st, (const InstanceRecord*)d_rec.get(), nt, (float4*)d_lo.get(), (float4*)d_hi.get());
+    if (nt) RT_HIP(ctx, hipMemcpyAsync(d_rec, trecs.data(), sizeof(InstanceRecord) * nt, hipMemcpyHostToDevice, st), "copy records");
+    RT_HIP(ctx, hipMemcpyAsync(d_seg, seg_start.data(), sizeof(uint32_t) * 2, hipMemcpyHostToDevice, st), "copy segments");
+    int rc = prepare_instances(st, d_rec, nt, d_lo, d_hi);
     if (rc) return hip_fail(ctx, hipError_t(rc), "prepare_instances");
     LbvhResult res;
     std::string err;
-    rc = lbvh_build(st, (const float4*)d_lo.get(), (const float4*)d_hi.get(), nt, (const uint32_t*)d_seg.get(),
-                    seg_start, kTlasLeafMax, ctx->collapse, ctx->treelets, &res, &err);
+    rc = lbvh_build(st, d_lo, d_hi, nt, d_seg, seg_start, kTlasLeafMax, ctx->collapse, ctx->treelets, sc, &res, &err);
     if (rc) return fail(ctx, rc == int(hipErrorOutOfMemory) ? RT_ERR_OUT_OF_MEMORY : RT_ERR_HIP, "TLAS build: " + err);
-    DevPtr perm(res.perm), seg_bounds(res.seg_bounds);
     te.nodes.reset(res.nodes);
     te.num_nodes = res.num_nodes;
     te.level_start = res.level_start;
@@ -676,8 +678,7 @@ int rt_build_tlas(rt_ctx* ctx, const rt_instance* d_instances, uint32_t count, r
     te.num_inst = count;
     te.num_tlas = nt;
     // records: TLAS leaf order first, then the flattened instances in caller order
-    rc = reorder_instances(st, (const InstanceRecord*)d_rec.get(), (const uint32_t*)perm.get(), nt,
-                           (InstanceRecord*)te.inst.get());
+    rc = reorder_instances(st, d_rec, res.perm, nt, (InstanceRecord*)te.inst.get());
     if (rc) return hip_fail(ctx, hipError_t(rc), "reorder_instances");
     std::vector<InstanceRecord> frecs(nf);
     std::vector<FlatSource> fsrc(nf);
@@ -695,40 +696,33 @@ int rt_build_tlas(rt_ctx* ctx, const rt_instance* d_instances, uint32_t count, r
     if (nf)
         RT_HIP(ctx, hipMemcpyAsync((InstanceRecord*)te.inst.get() + nt, frecs.data(), sizeof(InstanceRecord) * nf,
                                    hipMemcpyHostToDevice, st), "copy records");
-    RT_HIP(ctx, hipMemcpyAsync(te.bounds, seg_bounds.get(), sizeof(te.bounds), hipMemcpyDeviceToHost, st), "copy bounds");
+    RT_HIP(ctx, hipMemcpyAsync(te.bounds, res.seg_bounds, sizeof(te.bounds), hipMemcpyDeviceToHost, st), "copy bounds");
     if (nf) {
-        const uint32_t n = uint32_t(flat_total);
-        DevPtr d_src(dev_alloc<FlatSource>(nf, &e));
-        if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-        DevPtr d_tri_in(dev_alloc<float4>(3 * size_t(n) + 3, &e));
-        if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-        DevPtr d_flo(dev_alloc<float4>(n + 1, &e));
-        if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-        DevPtr d_fhi(dev_alloc<float4>(n + 1, &e));
-        if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-        DevPtr d_fseg(dev_alloc<uint32_t>(2, &e));
-        if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
+        const uint32_t n = fn;
+        FlatSource* d_src = sc.alloc<FlatSource>(nf);
+        float4* d_tri_in = sc.alloc<float4>(3 * size_t(n) + 3);
+        float4* d_flo = sc.alloc<float4>(n + 1);
+        float4* d_fhi = sc.alloc<float4>(n + 1);
+        uint32_t* d_fseg = sc.alloc<uint32_t>(2);
+        if (!d_src || !d_tri_in || !d_flo || !d_fhi || !d_fseg)
+            return fail(ctx, RT_ERR_OUT_OF_MEMORY, "flattened BVH build: out of device memory");
         std::vector<uint32_t> fseg = {0u, n};
-        RT_HIP(ctx, hipMemcpyAsync(d_src.get(), fsrc.data(), sizeof(FlatSource) * nf, hipMemcpyHostToDevice, st), "copy sources");
-        RT_HIP(ctx, hipMemcpyAsync(d_fseg.get(), fseg.data(), sizeof(uint32_t) * 2, hipMemcpyHostToDevice, st), "copy segments");
-        rc = gather_flat(st, (const FlatSource*)d_src.get(), nf, n, (float4*)d_tri_in.get(), (float4*)d_flo.get(),
-                         (float4*)d_fhi.get());
+        RT_HIP(ctx, hipMemcpyAsync(d_src, fsrc.data(), sizeof(FlatSource) * nf, hipMemcpyHostToDevice, st), "copy sources");
+        RT_HIP(ctx, hipMemcpyAsync(d_fseg, fseg.data(), sizeof(uint32_t) * 2, hipMemcpyHostToDevice, st), "copy segments");
+        rc = gather_flat(st, d_src, nf, n, d_tri_in, d_flo, d_fhi);
         if (rc) return hip_fail(ctx, hipError_t(rc), "gather_flat");
         LbvhResult fres;
-        rc = lbvh_build(st, (const float4*)d_flo.get(), (const float4*)d_fhi.get(), n, (const uint32_t*)d_fseg.get(),
-                        fseg, ctx->leaf_max, ctx->collapse, ctx->treelets, &fres, &err);
+        rc = lbvh_build(st, d_flo, d_fhi, n, d_fseg, fseg, ctx->leaf_max, ctx->collapse, ctx->treelets, sc, &fres, &err);
         if (rc) return fail(ctx, rc == int(hipErrorOutOfMemory) ? RT_ERR_OUT_OF_MEMORY : RT_ERR_HIP, "flattened BVH build: " + err);
-        DevPtr fperm(fres.perm), fseg_bounds(fres.seg_bounds);
         te.flat_nodes.reset(fres.nodes);
         te.flat_num_nodes = fres.num_nodes;
         te.flat_level_start = fres.level_start;
         te.flat_tris.reset(dev_alloc<float4>(3 * size_t(n) + 3, &e));
         if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
         te.flat_num_tris = n;
-        rc = reorder_triangles(st, (const float4*)d_tri_in.get(), (const uint32_t*)fperm.get(), n,
-                               (float4*)te.flat_tris.get());
+        rc = reorder_triangles(st, d_tri_in, fres.perm, n, (float4*)te.flat_tris.get());
         if (rc) return hip_fail(ctx, hipError_t(rc), "reorder_triangles");
-        RT_HIP(ctx, hipMemcpyAsync(te.flat_bounds, fseg_bounds.get(), sizeof(te.flat_bounds), hipMemcpyDeviceToHost, st), "copy bounds");
+        RT_HIP(ctx, hipMemcpyAsync(te.flat_bounds, fres.seg_bounds, sizeof(te.flat_bounds), hipMemcpyDeviceToHost, st), "copy bounds");
         RT_HIP(ctx, hipStreamSynchronize(st), "hipStreamSynchronize");
     }
     RT_HIP(ctx, hipStreamSynchronize(st), "hipStreamSynchronize");

@@ -9,6 +9,7 @@
 // whole batch and every segment is its own subtree.
 #pragma once
 
+#include <string>
 #include <vector>
 
 #include "common.h"
@@ -27,13 +28,33 @@ struct TriSegment {
     uint32_t _pad;
 };
 
-// Scratch and results of one build; device pointers are owned by the caller
-// (api.hip) so that they can be pooled.
+// Device scratch of a context's builds, one after another on its stream: one block that
+// the buffers of a build are cut from, kept between builds (forty allocations and
+// releases per build took longer than the kernels of a small scene).  A build begins it
+// with the bytes it expects (a buffer beyond them is allocated by itself) and ends it
+// after synchronising its stream.  A block above kScratchKeep is given back at the end
+// of the build, the others when the context is destroyed.
+struct ScratchPool {
+    static constexpr size_t kScratchKeep = size_t(1) << 30;
+    char* base = nullptr;
+    size_t cap = 0, used = 0;
+    std::vector<void*> extra;
+    ~ScratchPool();
+    void begin(size_t bytes);
+    void* alloc_bytes(size_t bytes);
+    template <class T> T* alloc(size_t count) { return static_cast<T*>(alloc_bytes(count * sizeof(T))); }
+    void end();
+};
+
+// bytes lbvh_build takes from the pool, about
+size_t lbvh_scratch_bytes(uint32_t n, uint32_t nseg);
+
+// Results of one build.
 struct LbvhResult {
-    QNode* nodes = nullptr;         // final (quantised) node array, exact size
+    QNode* nodes = nullptr;         // final (quantised) node array, exact size, owned by the caller
     uint32_t num_nodes = 0;
-    uint32_t* perm = nullptr;       // sorted position -> input primitive index
-    float* seg_bounds = nullptr;    // 6 floats per segment (padded root box)
+    const uint32_t* perm = nullptr; // sorted position -> input primitive index (scratch)
+    float* seg_bounds = nullptr;    // 6 floats per segment (padded root box; scratch)
     std::vector<uint32_t> level_start;  // nodes of tree level L: [level_start[L], level_start[L + 1])
 };
 
@@ -47,10 +68,12 @@ enum : uint32_t {
 // `nseg` segments (d_seg_start has nseg + 1 entries, on device and host).
 // Segment s's root is node s.  Leaves hold at most leaf_max primitives.
 // treelet_passes: bottom-up treelet restructurings of the binary tree before the
-// collapse (0: none).  Returns a hipError_t-compatible code.
+// collapse (0: none).  Scratch, perm and seg_bounds come from `scratch`.  Returns a
+// hipError_t-compatible code.
 int lbvh_build(hipStream_t stream, const float4* d_lo, const float4* d_hi, uint32_t n,
                const uint32_t* d_seg_start, const std::vector<uint32_t>& h_seg_start,
-               uint32_t leaf_max, uint32_t collapse, uint32_t treelet_passes, LbvhResult* out, std::string* err);
+               uint32_t leaf_max, uint32_t collapse, uint32_t treelet_passes, ScratchPool& scratch, LbvhResult* out,
+               std::string* err);
 
 // Triangle preparation for a BLAS batch: reads the caller's index and vertex
 // buffers, writes triangle records (input order) and boxes.  Sets *d_bad to 1 if an

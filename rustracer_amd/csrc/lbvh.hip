@@ -167,12 +167,6 @@ __device__ inline QNode quantize_node(const WideNode& w) {
     return q;
 }
 
-__global__ void k_quantize_nodes(const WideNode* in, uint32_t n, QNode* out) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    out[i] = quantize_node(in[i]);
-}
-
 __global__ void k_gather_flat(const FlatSource* src, uint32_t nsrc, uint32_t n, float4* tri, float4* lo, float4* hi) {
     uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
@@ -239,49 +233,83 @@ __global__ void k_init_bounds(uint32_t* bounds, uint32_t nseg) {
     bounds[i] = is_lo ? f2ord(INFINITY) : f2ord(-INFINITY);
 }
 
-__global__ void k_seg_bounds(const float4* lo, const float4* hi, uint32_t n, const uint32_t* seg_start, uint32_t nseg,
-                             uint32_t* bounds) {
-    uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    bool valid = p < n;
-    uint32_t seg = valid ? find_segment(seg_start, nseg, p) : 0;
-    float v[12];
-    if (valid) {
-        float4 l = lo[p], h = hi[p];
-        v[0] = 0.5f * (l.x + h.x); v[1] = 0.5f * (l.y + h.y); v[2] = 0.5f * (l.z + h.z);
-        v[3] = v[0]; v[4] = v[1]; v[5] = v[2];
-        v[6] = l.x; v[7] = l.y; v[8] = l.z;
-        v[9] = h.x; v[10] = h.y; v[11] = h.z;
-    } else {
-        for (int k = 0; k < 12; k++) {
-            bool is_lo = (k < 3) || (k >= 6 && k < 9);
-            v[k] = is_lo ? INFINITY : -INFINITY;
-        }
+constexpr uint32_t kBoundsItems = 16;  // most primitives per thread of k_seg_bounds
+// enough workgroups to fill the chip twice before a thread takes more than one
+inline uint32_t bounds_span(uint32_t n) {
+    return uint32_t(kBlock) * std::min(std::max(n / (uint32_t(kBlock) * 512u), 1u), kBoundsItems);
+}
+
+__device__ inline bool bound_is_lo(int k) { return k < 3 || (k >= 6 && k < 9); }
+__device__ inline void bounds_none(float v[12]) {
+#pragma unroll
+    for (int k = 0; k < 12; k++) v[k] = bound_is_lo(k) ? INFINITY : -INFINITY;
+}
+__device__ inline void bounds_add(float v[12], float4 l, float4 h) {
+    const float c[3] = {0.5f * (l.x + h.x), 0.5f * (l.y + h.y), 0.5f * (l.z + h.z)};
+    const float b[6] = {l.x, l.y, l.z, h.x, h.y, h.z};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        v[k] = fminf(v[k], c[k]);
+        v[3 + k] = fmaxf(v[3 + k], c[k]);
+        v[6 + k] = fminf(v[6 + k], b[k]);
+        v[9 + k] = fmaxf(v[9 + k], b[3 + k]);
     }
-    // wave-uniform segment: reduce in registers, one atomic per wave
-    uint32_t s0 = __shfl(seg, 0, 64);
-    bool uniform = __ballot(seg != s0 && valid) == 0ull;
-    if (uniform) {
-        for (int k = 0; k < 12; k++) {
-            bool is_lo = (k < 3) || (k >= 6 && k < 9);
-            float x = v[k];
-            for (int o = 32; o > 0; o >>= 1) {
-                float y = __shfl_xor(x, o, 64);
-                x = is_lo ? fminf(x, y) : fmaxf(x, y);
-            }
-            v[k] = x;
+}
+__device__ inline void bounds_wave(float v[12]) {
+#pragma unroll
+    for (int k = 0; k < 12; k++)
+        for (int o = 32; o > 0; o >>= 1) {
+            const float y = __shfl_xor(v[k], o, 64);
+            v[k] = bound_is_lo(k) ? fminf(v[k], y) : fmaxf(v[k], y);
         }
-        if (__lane_id() == 0 && __ballot(valid) != 0ull) {
-            for (int k = 0; k < 12; k++) {
-                bool is_lo = (k < 3) || (k >= 6 && k < 9);
-                if (is_lo) atomicMin(&bounds[12 * s0 + k], f2ord(v[k]));
-                else atomicMax(&bounds[12 * s0 + k], f2ord(v[k]));
-            }
+}
+__device__ inline void bounds_atomic(uint32_t* b, int k, float v) {
+    if (bound_is_lo(k)) atomicMin(&b[k], f2ord(v));
+    else atomicMax(&b[k], f2ord(v));
+}
+
+// A workgroup reduces up to 4096 primitives before its 12 atomics: all of one segment's
+// atomics go to the same 12 words, one after another (one set per wave took 4.2 ms for a
+// segment of 2M primitives, this 87 us; 4096 for 5,120 primitives as well were 50 us).
+__global__ __launch_bounds__(kBlock) void k_seg_bounds(const float4* lo, const float4* hi, uint32_t n,
+                                                        const uint32_t* seg_start, uint32_t nseg, uint32_t span,
+                                                        uint32_t* bounds) {
+    __shared__ float s_v[kBlock / 64][12];
+    const uint32_t base = blockIdx.x * span;
+    const uint32_t end = base + min(span, n - base);
+    const uint32_t s0 = find_segment(seg_start, nseg, base);
+    float v[12];
+    if (s0 == find_segment(seg_start, nseg, end - 1u)) {
+        bounds_none(v);
+        for (uint32_t p = base + threadIdx.x; p < end; p += kBlock) bounds_add(v, lo[p], hi[p]);
+        bounds_wave(v);
+        if ((threadIdx.x & 63u) == 0u)
+            for (int k = 0; k < 12; k++) s_v[threadIdx.x >> 6][k] = v[k];
+        __syncthreads();
+        if (threadIdx.x < 12u) {
+            const int k = int(threadIdx.x);
+            float x = s_v[0][k];
+            for (int w = 1; w < kBlock / 64; w++) x = bound_is_lo(k) ? fminf(x, s_v[w][k]) : fmaxf(x, s_v[w][k]);
+            bounds_atomic(bounds + 12 * size_t(s0), k, x);
         }
-    } else if (valid) {
-        for (int k = 0; k < 12; k++) {
-            bool is_lo = (k < 3) || (k >= 6 && k < 9);
-            if (is_lo) atomicMin(&bounds[12 * seg + k], f2ord(v[k]));
-            else atomicMax(&bounds[12 * seg + k], f2ord(v[k]));
+        return;
+    }
+    // several segments: a wave at a time
+    for (uint32_t row = base; row < end; row += kBlock) {
+        const uint32_t p = row + threadIdx.x;
+        const bool valid = p < end;
+        const uint32_t seg = valid ? find_segment(seg_start, nseg, p) : 0u;
+        bounds_none(v);
+        if (valid) bounds_add(v, lo[p], hi[p]);
+        const uint64_t live = __ballot(valid);
+        if (!live) continue;  // the wave's row is past the end
+        const uint32_t w0 = __shfl(seg, 0, 64);  // lane 0 is valid when any lane is
+        if (__ballot(valid && seg != w0) == 0ull) {
+            bounds_wave(v);
+            if (__lane_id() == 0)
+                for (int k = 0; k < 12; k++) bounds_atomic(bounds + 12 * size_t(w0), k, v[k]);
+        } else if (valid) {
+            for (int k = 0; k < 12; k++) bounds_atomic(bounds + 12 * size_t(seg), k, v[k]);
         }
     }
 }
@@ -413,6 +441,39 @@ __global__ __launch_bounds__(kBlock) void k_rs_scatter(const uint64_t* kin, cons
     }
 }
 
+// Sort of at most kRankMax keys in one launch: the position of a key is the number of
+// keys below it, counting equal keys of smaller index (the stable order of the radix
+// passes).  kRankSlices lanes share a key's count.  Kernel time against that of the 24 to
+// 40 radix launches: 22 us to 120 us at 5,120 keys, 66 to 167 at 16,384; at 32,768 the
+// n^2 compares take 260 us, the radix passes 170.
+constexpr uint32_t kRankMax = 16384;
+constexpr int kRankKeys = 64, kRankSlices = 16;
+
+__global__ __launch_bounds__(kRankKeys * kRankSlices) void k_rank_sort(const uint64_t* kin, const uint32_t* vin,
+                                                                      uint32_t n, uint64_t* kout, uint32_t* vout) {
+    __shared__ uint32_t s_rank[kRankKeys];
+    const uint32_t e = threadIdx.x & (kRankKeys - 1), slice = threadIdx.x / kRankKeys;
+    const uint32_t i = blockIdx.x * kRankKeys + e;
+    if (threadIdx.x < kRankKeys) s_rank[threadIdx.x] = 0u;
+    __syncthreads();
+    const uint64_t key = i < n ? kin[i] : 0ull;
+    const uint32_t per = (n + kRankSlices - 1) / kRankSlices;
+    const uint32_t j0 = min(slice * per, n), j1 = min(j0 + per, n);
+    uint32_t c = 0;
+#pragma unroll 8
+    for (uint32_t j = j0; j < j1; j++) {
+        const uint64_t k = kin[j];  // the same address in every lane of a wave
+        c += (k < key || (k == key && j < i)) ? 1u : 0u;
+    }
+    atomicAdd(&s_rank[e], c);
+    __syncthreads();
+    if (slice == 0 && i < n) {
+        const uint32_t r = s_rank[e];  // below n: the counts of n keys are a permutation
+        kout[r] = key;
+        vout[r] = vin[i];
+    }
+}
+
 int exclusive_scan(hipStream_t st, uint32_t* d, uint32_t m, uint32_t* tmp, uint32_t tmp_cap) {
     uint32_t nb = blocks_for(m, kScanPerBlock);
     if (nb > tmp_cap) return int(hipErrorInvalidValue);
@@ -437,8 +498,13 @@ __device__ inline int delta(const uint64_t* k, int n, int i, int j) {
 
 __global__ void k_karras(const uint64_t* keys, int n, uint32_t* left, uint32_t* right, uint32_t* first,
                          uint32_t* last, uint32_t* parent_int, uint32_t* parent_leaf, const uint32_t* seg_start,
-                         uint32_t nseg, int seg_shift, uint32_t* seg_root) {
+                         uint32_t nseg, int seg_shift, uint32_t* seg_root, uint32_t* is_root, uint32_t* split_node) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
+    // the root of the whole tree (node 0, or the only leaf) has no parent
+    if (i == 0) {
+        if (n == 1) parent_leaf[0] = kEmpty;
+        else parent_int[0] = kEmpty;
+    }
     if (i >= n - 1) return;
     int d = (delta(keys, n, i, i + 1) - delta(keys, n, i, i - 1)) >= 0 ? 1 : -1;
     int dmin = delta(keys, n, i, i - d);
@@ -460,27 +526,15 @@ __global__ void k_karras(const uint64_t* keys, int n, uint32_t* left, uint32_t* 
     uint32_t rc = (hi == gamma + 1) ? (kLeafBit | uint32_t(gamma + 1)) : uint32_t(gamma + 1);
     left[i] = lc;
     right[i] = rc;
+    split_node[gamma] = i;  // the node that parts leaf gamma from gamma + 1
     first[i] = lo;
     last[i] = hi;
     if (lc & kLeafBit) parent_leaf[gamma] = i; else parent_int[gamma] = i;
     if (rc & kLeafBit) parent_leaf[gamma + 1] = i; else parent_int[gamma + 1] = i;
     uint32_t seg = uint32_t(keys[lo] >> seg_shift);
-    if (seg < nseg && uint32_t(lo) == seg_start[seg] && uint32_t(hi) + 1 == seg_start[seg + 1]) seg_root[seg] = i;
-}
-
-__global__ void k_single_roots(const uint32_t* seg_start, uint32_t nseg, uint32_t* seg_root) {
-    uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nseg) return;
-    uint32_t c = seg_start[s + 1] - seg_start[s];
-    if (c == 1) seg_root[s] = kLeafBit | seg_start[s];
-    else if (c == 0) seg_root[s] = kEmpty;
-}
-
-__global__ void k_mark_roots(const uint32_t* seg_root, uint32_t nseg, uint32_t* is_root) {
-    uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nseg) return;
-    uint32_t r = seg_root[s];
-    if (r != kEmpty && !(r & kLeafBit)) is_root[r] = 1u;
+    const bool root = seg < nseg && uint32_t(lo) == seg_start[seg] && uint32_t(hi) + 1 == seg_start[seg + 1];
+    is_root[i] = root ? 1u : 0u;
+    if (root) seg_root[seg] = i;
 }
 
 // --------------------------------------------------------------- box fit
@@ -512,258 +566,508 @@ constexpr float kSahTriCost = 0.6f;
 //   bits 8..9   i* - 2 of the node's own wide node, bits 10..11 its k*
 __device__ inline uint32_t dec_slots(uint32_t d, int i) { return (d >> (2 * (i - 1))) & 3u; }
 
-struct SahArgs {
-    float4* cost;     // per binary node: C(n, 1..4)
-    uint32_t* dec;    // per binary node: decision word
-    const uint32_t* first;
-    const uint32_t* last;
-    uint32_t leaf_max;
-};
-
-// C(r, 1..4) of a child reference: a primitive costs one triangle test wherever it goes
-__device__ inline float4 child_cost(uint32_t r, const SahArgs& sa, float3 l, float3 h) {
-    if (r & kLeafBit) {
-        float c = kSahTriCost * half_area(l, h);
-        return make_float4(c, c, c, c);
+// Exclusive sum over the workgroup; `total` gets the sum of all.
+template <int T> __device__ inline uint32_t block_exclusive(uint32_t v, uint32_t* s_wave, uint32_t& total) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint32_t x = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= uint32_t(o)) x += y;
     }
-    return sa.cost[r];
+    __syncthreads();
+    if (lane == 63u) s_wave[wave] = x;
+    __syncthreads();
+    uint32_t before = 0;
+    total = 0;
+    for (uint32_t w = 0; w < uint32_t(T) / 64u; w++) {
+        if (w < wave) before += s_wave[w];
+        total += s_wave[w];
+    }
+    return before + x - v;
 }
 
-__device__ inline void sah_node(uint32_t node, uint32_t a, uint32_t b, float3 la, float3 ha, float3 lb, float3 hb,
-                                float3 l, float3 h, const SahArgs& sa) {
-    const float4 ca4 = child_cost(a, sa, la, ha), cb4 = child_cost(b, sa, lb, hb);
+// ------------------------------------------------- bottom-up passes
+// Boxes, treelet restructuring and SAH costs are computed bottom-up: of the two threads
+// that reach a node from below, the second handles it.  Done over the whole tree in
+// global memory, every node costs an agent-scope acquire-release, which writes back and
+// invalidates caches (8.3 ms for the box fit alone of 2M primitives, 15.8 ms for a
+// treelet pass).  So the tree is taken in tiles of consecutive leaves: the nodes whose
+// leaves lie in one tile of kTile leaves are handled by one workgroup, in LDS, all passes
+// in one launch; then those of a tile kFan times as large, over the subtrees that the
+// smaller tiles left, and so on (k_tree_level).  A subtree of a smaller tile is not
+// opened again, so a treelet does not reach across it: node visits per ray are the same
+// to 0.1 %.  For 2M primitives both treelet passes, boxes and SAH costs take
+// 2.0 ms, against 39.8 ms.
+constexpr int kTile = 512;        // leaves of a first tile, and its threads
+constexpr int kTileRefs = 768;    // subtrees a larger tile can hold
+constexpr int kTileThreads = 256; // threads of a larger tile
+// A tile leaves about 15 subtrees, so 16 tiles make a larger one; where a tile turns out to
+// hold more than kTileRefs, the build starts over with 4, whose subtrees always fit.
+constexpr uint32_t kFan = 16, kFanSafe = 4;
+// Subtrees of unfinished segments that a tile leaves: they hang off the tree's paths to
+// the tile's first and last leaf, one per node of a path, and a path is shorter than the
+// key and index bits together.
+constexpr uint32_t kTileRoots = 192;
+static_assert(kFanSafe * kTileRoots <= uint32_t(kTileRefs), "four tiles' subtrees fit");
+constexpr uint32_t kOverflowNodes = 1u, kOverflowRoots = 2u, kOverflowFan = 4u;  // bits of the overflow word
+
+// SAH costs C(n, 1..4) of a node from its children's costs and boxes; the decision word
+// is returned in d.
+__device__ inline float4 sah_costs(float4 ca4, float4 cb4, float area, uint32_t count, uint32_t leaf_max, uint32_t& d) {
     const float ca[5] = {0.f, ca4.x, ca4.y, ca4.z, ca4.w}, cb[5] = {0.f, cb4.x, cb4.y, cb4.z, cb4.w};
     float dist[5];
     uint32_t kbest[5];
+#pragma unroll
     for (int i = 2; i <= 4; i++) {
         dist[i] = INFINITY;
         kbest[i] = 1;
+#pragma unroll
         for (int k = 1; k < i; k++) {
             const float c = ca[k] + cb[i - k];
             if (c < dist[i]) { dist[i] = c; kbest[i] = uint32_t(k); }
         }
     }
-    int istar = 2;
+    uint32_t istar = 2, kstar = kbest[2];
+    float dmin = dist[2];
+#pragma unroll
     for (int i = 3; i <= 4; i++)
-        if (dist[i] < dist[istar]) istar = i;
-    const float area = half_area(l, h);
-    const float c_int = kSahNodeCost * area + dist[istar];
-    const uint32_t cnt = sa.last[node] - sa.first[node] + 1u;
-    const float c_leaf = cnt <= sa.leaf_max ? kSahTriCost * float(cnt) * area : INFINITY;
+        if (dist[i] < dmin) { dmin = dist[i]; istar = uint32_t(i); kstar = kbest[i]; }
+    const float c_int = kSahNodeCost * area + dmin;
+    const float c_leaf = count <= leaf_max ? kSahTriCost * float(count) * area : INFINITY;
     float c[5];
-    uint32_t d = 0;
+    d = 0;
     if (c_int < c_leaf) { c[1] = c_int; d |= 1u; } else { c[1] = c_leaf; }
+#pragma unroll
     for (int i = 2; i <= 4; i++) {
         if (dist[i] < c[i - 1]) { c[i] = dist[i]; d |= kbest[i] << (2 * (i - 1)); }
         else c[i] = c[i - 1];
     }
-    d |= uint32_t(istar - 2) << 8;
-    d |= kbest[istar] << 10;
-    sa.cost[node] = make_float4(c[1], c[2], c[3], c[4]);
-    sa.dec[node] = d;
+    d |= (istar - 2u) << 8;
+    d |= kstar << 10;
+    return make_float4(c[1], c[2], c[3], c[4]);
+}
+// a primitive costs one triangle test wherever it goes
+__device__ inline float4 sah_leaf(float3 l, float3 h) {
+    const float c = kSahTriCost * half_area(l, h);
+    return make_float4(c, c, c, c);
 }
 
-template <bool kSah>
-__global__ void k_fit(const float4* lo, const float4* hi, const uint32_t* perm, int n, const uint32_t* left,
-                      const uint32_t* right, const uint32_t* parent_int, const uint32_t* parent_leaf,
-                      const uint32_t* is_root, uint32_t* visits, float4* nlo, float4* nhi, SahArgs sa) {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    uint32_t node = parent_leaf[p];
-    while (node != kEmpty) {
-        // the second child to arrive computes the union (and the SAH costs); acq_rel
-        // makes the first child's box and costs visible
-        uint32_t prev = __hip_atomic_fetch_add(&visits[node], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (prev == 0u) return;
-        float3 l0, h0, l1, h1;
-        const uint32_t a = left[node], b = right[node];
-        load_box(a, lo, hi, perm, nlo, nhi, l0, h0);
-        load_box(b, lo, hi, perm, nlo, nhi, l1, h1);
-        float3 l = fmin3(l0, l1), h = fmax3(h0, h1);
-        nlo[node] = make_float4(l.x, l.y, l.z, 0.f);
-        nhi[node] = make_float4(h.x, h.y, h.z, 0.f);
-        if (kSah) sah_node(node, a, b, l0, h0, l1, h1, l, h, sa);
-        if (is_root[node]) return;
-        node = parent_int[node];
-    }
-}
-
-// ------------------------------------------------- treelet restructuring
-// Karras & Aila, "Fast Parallel Construction of High-Quality Bounding Volume
-// Hierarchies" (HPG 2013): bottom up, each node of the binary tree gathers a
-// treelet of up to kTreeletLeaves leaves (it opens the largest-area internal leaf
-// until that many are gathered), finds the binary tree over those leaves of least
-// surface-area-heuristic cost by a dynamic program over the leaf subsets, and
-// rebuilds the treelet that way when that is cheaper, reusing its internal nodes.
-// Cost of a subtree: kTreeletNodeCost * A(n) + C(left) + C(right), and
-// kTreeletTriCost * A(p) for a primitive.  Subtrees stop covering contiguous runs
-// of the sorted primitives; a renumbering in depth-first order restores that
-// before the collapse.
-// Five leaves: 3^5 = 243 steps of the subset program per node.  On a 2M-triangle
-// scene, seven leaves (2187 steps) took 233 ms per build against 109 ms for five,
-// for 10.12 against 10.18 node visits per ray (10.71 without restructuring).
+// Treelet restructuring (Karras & Aila, "Fast Parallel Construction of High-Quality
+// Bounding Volume Hierarchies", HPG 2013): bottom up, each node of the binary tree gathers
+// a treelet of up to kTreeletLeaves leaves (it opens the largest-area internal leaf until
+// that many are gathered), finds the binary tree over those leaves of least
+// surface-area-heuristic cost by a dynamic program over the leaf subsets, and rebuilds
+// the treelet that way when that is cheaper, reusing its internal nodes.  Cost of a
+// subtree: kTreeletNodeCost * A(n) + C(left) + C(right), and kTreeletTriCost * A(p) for a
+// primitive.  Subtrees stop covering contiguous runs of the sorted primitives; a
+// renumbering in depth-first order restores that before the collapse.
+// Five leaves: 90 splits of 26 subsets per node, all in registers (every index of the
+// arrays below is a constant once unrolled).  Seven leaves gave 10.12 against 10.18 node
+// visits per ray (10.71 without restructuring) for nine times the splits.
 constexpr int kTreeletLeaves = 5;
 constexpr float kTreeletNodeCost = 1.2f;
 constexpr float kTreeletTriCost = 1.0f;
 constexpr int kMaxWalk = 1 << 16;  // bound of the walks up the binary tree
 
-struct TreeletArgs {
-    const float4* lo;
+struct TreeRef {  // what a pass needs of a node or leaf
+    float3 l, h;
+    float c;     // treelet cost
+    uint32_t n;  // primitives
+};
+
+template <class T> __device__ inline T pick5(const T (&a)[5], uint32_t i) {
+    T r = a[0];
+#pragma unroll
+    for (uint32_t k = 1; k < 5; k++) r = i == k ? a[k] : r;
+    return r;
+}
+
+// box, cost and primitive count of `node` from its children, stored; the cost and count
+// are returned
+template <class Store> __device__ inline float tree_refresh(Store& st, uint32_t node, uint32_t& count) {
+    const TreeRef a = st.get(st.left(node)), b = st.get(st.right(node));
+    TreeRef r;
+    r.l = fmin3(a.l, b.l);
+    r.h = fmax3(a.h, b.h);
+    r.c = kTreeletNodeCost * half_area(r.l, r.h) + a.c + b.c;
+    r.n = a.n + b.n;
+    st.put(node, r);
+    count = r.n;
+    return r.c;
+}
+
+template <class Store> __device__ inline void treelet_optimize(Store& st, uint32_t node, float cur) {
+    constexpr int M = kTreeletLeaves;
+    static_assert(M == 5, "the subset words below hold 5-bit subsets");
+    uint32_t leaf[M], inner[M];
+    TreeRef lf[M];
+    leaf[0] = st.left(node);
+    leaf[1] = st.right(node);
+    lf[0] = st.get(leaf[0]);
+    lf[1] = st.get(leaf[1]);
+    inner[0] = node;
+    uint32_t m = 2;
+#pragma unroll
+    for (int k = 2; k < M; k++) {
+        leaf[k] = leaf[0];
+        lf[k] = lf[0];
+        inner[k - 1] = node;
+    }
+    inner[M - 1] = node;
+#pragma unroll
+    for (int k = 2; k < M; k++) {
+        if (m != uint32_t(k)) break;
+        int best = -1;
+        float best_a = -1.f;
+#pragma unroll
+        for (int j = 0; j < k; j++) {
+            const float ar = half_area(lf[j].l, lf[j].h);
+            if (!st.is_leaf(leaf[j]) && ar > best_a) { best_a = ar; best = j; }
+        }
+        if (best < 0) break;
+        const uint32_t x = pick5(leaf, uint32_t(best));
+        inner[k - 1] = x;
+        const uint32_t xl = st.left(x), xr = st.right(x);
+        const TreeRef tl = st.get(xl), tr = st.get(xr);
+#pragma unroll
+        for (int j = 0; j < k; j++)
+            if (j == best) {
+                leaf[j] = xl;
+                lf[j] = tl;
+            }
+        leaf[k] = xr;
+        lf[k] = tr;
+        m = uint32_t(k) + 1u;
+    }
+    if (m < 3u) return;
+    // least cost of a binary tree over each subset S of the leaves; part(S), the subset of
+    // S that goes to the left child, in 5 bits of pw
+    const uint32_t full = (1u << m) - 1u;
+    float cost[1 << M];
+    uint64_t pw[3] = {0ull, 0ull, 0ull};
+#pragma unroll
+    for (int k = 0; k < M; k++) cost[1 << k] = lf[k].c;
+    float all = INFINITY;
+#pragma unroll
+    for (uint32_t S = 3; S < (1u << M); S++) {
+        if ((S & (S - 1u)) == 0u) continue;
+        if (S > full) break;
+        float3 l = mk3(INFINITY, INFINITY, INFINITY), h = mk3(-INFINITY, -INFINITY, -INFINITY);
+#pragma unroll
+        for (int i = 0; i < M; i++)
+            if ((S >> i) & 1u) { l = fmin3(l, lf[i].l); h = fmax3(h, lf[i].h); }
+        const uint32_t low = S & (0u - S);
+        float best = INFINITY;
+        uint32_t bp = low;
+#pragma unroll
+        for (uint32_t P = 1; P < S; P++) {  // the left part holds the lowest leaf
+            if ((P & S) != P || !(P & low)) continue;
+            const float c = cost[P] + cost[S ^ P];
+            if (c < best) { best = c; bp = P; }
+        }
+        cost[S] = kTreeletNodeCost * half_area(l, h) + best;
+        pw[S / 12] |= uint64_t(bp) << (5 * (S % 12));
+        if (S == full) all = cost[S];
+    }
+    if (!(all < 0.9999f * cur)) return;
+    // rebuild: internal node inner[k] takes subset k of the queue, top down
+    uint32_t queue = full, next = 1;
+#pragma unroll
+    for (int k = 0; k < M - 1; k++) {
+        if (uint32_t(k) >= next) break;
+        const uint32_t S = (queue >> (5 * k)) & 31u;
+        const uint32_t w = S / 12u;
+        const uint32_t P = uint32_t((w == 0u ? pw[0] : (w == 1u ? pw[1] : pw[2])) >> (5u * (S - 12u * w))) & 31u;
+        const uint32_t sub[2] = {P, S ^ P};
+        uint32_t ref[2];
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            if ((sub[c] & (sub[c] - 1u)) == 0u) {
+                ref[c] = pick5(leaf, uint32_t(__ffs(int(sub[c]))) - 1u);
+            } else {
+                ref[c] = pick5(inner, next);
+                queue |= sub[c] << (5u * next);
+                next++;
+            }
+            st.set_parent(ref[c], inner[k]);
+        }
+        st.set_children(inner[k], ref[0], ref[1]);
+    }
+    // children before parents (a child's place in the queue is behind its parent's)
+    uint32_t count;
+#pragma unroll
+    for (int k = M - 2; k >= 0; k--)
+        if (uint32_t(k) < next) (void)tree_refresh(st, inner[k], count);
+}
+
+struct TreeArgs {
+    const float4* lo;   // primitive boxes
     const float4* hi;
-    const uint32_t* perm;
+    const uint32_t* perm;  // sorted position -> primitive
+    const uint64_t* keys;  // sorted
+    int seg_shift;
+    const uint32_t* seg_start;
+    const uint32_t* first;  // leaf range of each node as the radix tree was emitted
+    const uint32_t* last;
+    const uint32_t* split_node;
     uint32_t* left;
     uint32_t* right;
     uint32_t* parent_int;
     uint32_t* parent_leaf;
-    const uint32_t* is_root;
-    uint32_t* visits;
-    float4* nlo;   // .w: the subtree's cost
+    float4* nlo;     // node boxes; nlo.w: treelet cost
     float4* nhi;
-    uint32_t* cnt;  // primitives under each internal node
-    const uint32_t* seg_start;
-    uint32_t nseg;
+    uint32_t* cnt;   // primitives under each node
+    float4* cost;    // C(n, 1..4) (SAH collapse)
+    uint32_t* dec;   // decision words (SAH collapse)
+    uint32_t* overflow;
+    uint32_t n;
+    uint32_t passes;   // treelet passes
+    uint32_t leaf_max;
+    uint32_t sah;
 };
 
-__device__ inline void treelet_ref(const TreeletArgs& a, uint32_t r, float3& l, float3& h, float& c, uint32_t& n) {
-    if (r & kLeafBit) {
-        const uint32_t s = a.perm[r & ~kLeafBit];
-        l = xyz(a.lo[s]);
-        h = xyz(a.hi[s]);
-        c = kTreeletTriCost * half_area(l, h);
-        n = 1u;
+// The subtrees ("entities", 0..C-1, in leaf order) and nodes (C..2C-1) of one tile in LDS.
+// Node k is the one whose split lies between entities k and k + 1.
+template <int C> struct TileStore {
+    static constexpr uint32_t kNone = 0xFFFFu;
+    float lo[3][2 * C], hi[3][2 * C];
+    float cost[2 * C];
+    uint32_t cnt[2 * C];
+    uint32_t ref[C];   // entity: kLeafBit | leaf position, or the subtree's root node
+    uint32_t id[C];    // node id (kEmpty: the split's node is not of this tile)
+    uint16_t child[2][C], parent[2 * C];
+    uint32_t seen[C / 32];
+
+    __device__ bool is_leaf(uint32_t e) const { return e < uint32_t(C); }
+    __device__ uint32_t left(uint32_t e) const { return child[0][e - C]; }
+    __device__ uint32_t right(uint32_t e) const { return child[1][e - C]; }
+    __device__ TreeRef get(uint32_t e) const {
+        TreeRef r;
+        r.l = mk3(lo[0][e], lo[1][e], lo[2][e]);
+        r.h = mk3(hi[0][e], hi[1][e], hi[2][e]);
+        r.c = cost[e];
+        r.n = cnt[e];
+        return r;
+    }
+    __device__ void put(uint32_t e, const TreeRef& r) {
+        lo[0][e] = r.l.x; lo[1][e] = r.l.y; lo[2][e] = r.l.z;
+        hi[0][e] = r.h.x; hi[1][e] = r.h.y; hi[2][e] = r.h.z;
+        cost[e] = r.c;
+        cnt[e] = r.n;
+    }
+    __device__ void set_children(uint32_t e, uint32_t a, uint32_t b) {
+        child[0][e - C] = uint16_t(a);
+        child[1][e - C] = uint16_t(b);
+    }
+    __device__ void set_parent(uint32_t e, uint32_t p) { parent[e] = uint16_t(p); }
+    // the second thread to arrive at a node handles it; workgroup scope: what the first one
+    // wrote, to LDS or through this CU's cache, is visible
+    __device__ bool second(uint32_t e) {
+        const uint32_t k = e - C, bit = 1u << (k & 31u);
+        return (__hip_atomic_fetch_or(&seen[k >> 5], bit, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) & bit) != 0u;
+    }
+};
+
+// One level: tile blockIdx.x of `size` leaves, T threads.  kFirst: its entities are the
+// leaves, else the subtrees that `fan` tiles of the level before left (roots_in,
+// kTileRoots a tile).
+template <int C, int T, bool kFirst>
+__global__ __launch_bounds__(T, 4) void k_tree_level(TreeArgs a, uint32_t size, uint32_t fan, const uint32_t* roots_in,
+                                                     const uint32_t* count_in, uint32_t tiles_in, uint32_t* roots_out,
+                                                     uint32_t* count_out) {
+    using Store = TileStore<C>;
+    __shared__ Store ts;
+    __shared__ uint32_t s_wave[T / 64];
+    const uint32_t t = threadIdx.x, n = a.n;
+    const uint32_t base = blockIdx.x * size, end = base + min(size, n - base);
+    uint32_t* const lastpos = reinterpret_cast<uint32_t*>(ts.cost + C);  // until the node costs are written
+    // entities
+    uint32_t ne = 0;
+    if (kFirst) {
+        ne = end - base;
+        for (uint32_t e = t; e < ne; e += T) ts.ref[e] = kLeafBit | (base + e);
     } else {
-        const float4 lw = a.nlo[r];
-        l = xyz(lw);
-        h = xyz(a.nhi[r]);
-        c = lw.w;
-        n = a.cnt[r];
-    }
-}
-
-// box, cost and primitive count of `node` from its children; returns the cost
-__device__ inline float treelet_refresh(const TreeletArgs& a, uint32_t node, uint32_t* count) {
-    float3 l0, h0, l1, h1;
-    float c0, c1;
-    uint32_t n0, n1;
-    treelet_ref(a, a.left[node], l0, h0, c0, n0);
-    treelet_ref(a, a.right[node], l1, h1, c1, n1);
-    const float3 l = fmin3(l0, l1), h = fmax3(h0, h1);
-    const float c = kTreeletNodeCost * half_area(l, h) + c0 + c1;
-    a.nlo[node] = make_float4(l.x, l.y, l.z, c);
-    a.nhi[node] = make_float4(h.x, h.y, h.z, 0.f);
-    a.cnt[node] = n0 + n1;
-    *count = n0 + n1;
-    return c;
-}
-
-__device__ inline void treelet_set_parent(const TreeletArgs& a, uint32_t child, uint32_t parent) {
-    if (child & kLeafBit) a.parent_leaf[child & ~kLeafBit] = parent;
-    else a.parent_int[child] = parent;
-}
-
-__device__ void treelet_optimize(const TreeletArgs& a, uint32_t node, float cur) {
-    uint32_t leaf[kTreeletLeaves], inner[kTreeletLeaves - 1];
-    float3 ll[kTreeletLeaves], lh[kTreeletLeaves];
-    float lc[kTreeletLeaves];
-    uint32_t ln;
-    leaf[0] = a.left[node];
-    leaf[1] = a.right[node];
-    treelet_ref(a, leaf[0], ll[0], lh[0], lc[0], ln);
-    treelet_ref(a, leaf[1], ll[1], lh[1], lc[1], ln);
-    inner[0] = node;
-    int m = 2;
-    while (m < kTreeletLeaves) {
-        int best = -1;
-        float best_a = -1.f;
-        for (int j = 0; j < m; j++) {
-            if (leaf[j] & kLeafBit) continue;
-            const float ar = half_area(ll[j], lh[j]);
-            if (ar > best_a) { best_a = ar; best = j; }
-        }
-        if (best < 0) break;
-        const uint32_t x = leaf[best];
-        inner[m - 1] = x;
-        leaf[best] = a.left[x];
-        leaf[m] = a.right[x];
-        treelet_ref(a, leaf[best], ll[best], lh[best], lc[best], ln);
-        treelet_ref(a, leaf[m], ll[m], lh[m], lc[m], ln);
-        m++;
-    }
-    if (m < 3) return;
-    // least cost of a binary tree over each subset of the leaves; part[S] is the
-    // subset of S that goes to the left child
-    float cost[1 << kTreeletLeaves];
-    uint8_t part[1 << kTreeletLeaves];
-    const uint32_t full = (1u << m) - 1u;
-    for (uint32_t S = 1; S <= full; S++) {
-        if ((S & (S - 1u)) == 0u) {
-            cost[S] = lc[__ffs(S) - 1];
-            continue;
-        }
-        float3 l = mk3(INFINITY, INFINITY, INFINITY), h = mk3(-INFINITY, -INFINITY, -INFINITY);
-        for (int i = 0; i < m; i++)
-            if ((S >> i) & 1u) { l = fmin3(l, ll[i]); h = fmax3(h, lh[i]); }
-        const uint32_t low = S & (0u - S), rest = S ^ low;
-        float best = INFINITY;
-        uint32_t bp = low;
-        for (uint32_t q = rest;; q = (q - 1u) & rest) {
-            const uint32_t P = q | low;
-            if (P != S) {
-                const float c = cost[P] + cost[S ^ P];
-                if (c < best) { best = c; bp = P; }
+        // an earlier level that did not finish: its tiles' subtrees are missing (read once,
+        // so that every thread decides alike)
+        if (t == 0) s_wave[0] = *a.overflow;
+        __syncthreads();
+        if (s_wave[0]) return;
+        __syncthreads();
+        for (uint32_t k = 0; k < fan; k++) {
+            const uint32_t tile = blockIdx.x * fan + k;
+            const uint32_t c = tile < tiles_in ? count_in[tile] : 0u;
+            if (ne + c > uint32_t(C)) {  // the same for every thread
+                if (t == 0) {
+                    atomicOr(a.overflow, kOverflowFan);
+                    if (roots_out) count_out[blockIdx.x] = 0u;
+                }
+                return;
             }
-            if (q == 0u) break;
+            for (uint32_t i = t; i < c; i += T) ts.ref[ne + i] = roots_in[tile * kTileRoots + i];
+            ne += c;
         }
-        cost[S] = kTreeletNodeCost * half_area(l, h) + best;
-        part[S] = uint8_t(bp);
     }
-    if (!(cost[full] < 0.9999f * cur)) return;
-    // rebuild top down, handing out the treelet's internal nodes in order
-    uint32_t st_set[kTreeletLeaves], st_node[kTreeletLeaves], order[kTreeletLeaves - 1];
-    int sp = 0, no = 0, next = 1;
-    st_set[sp] = full;
-    st_node[sp++] = node;
-    while (sp > 0) {
-        sp--;
-        const uint32_t S = st_set[sp], X = st_node[sp];
-        order[no++] = X;
-        const uint32_t sub[2] = {uint32_t(part[S]), S ^ uint32_t(part[S])};
-        uint32_t ref[2];
-        for (int c = 0; c < 2; c++) {
-            if ((sub[c] & (sub[c] - 1u)) == 0u) {
-                ref[c] = leaf[__ffs(sub[c]) - 1];
+    __syncthreads();
+    for (uint32_t e = t; e < ne; e += T) {
+        const uint32_t r = ts.ref[e];
+        TreeRef x;
+        if (r & kLeafBit) {
+            const uint32_t pos = r & ~kLeafBit, s = a.perm[pos];
+            x.l = xyz(a.lo[s]);
+            x.h = xyz(a.hi[s]);
+            x.c = kTreeletTriCost * half_area(x.l, x.h);
+            x.n = 1u;
+            lastpos[e] = pos;
+        } else {
+            const float4 lw = a.nlo[r];
+            x.l = xyz(lw);
+            x.h = xyz(a.nhi[r]);
+            x.c = lw.w;
+            x.n = a.cnt[r];
+            lastpos[e] = a.last[r];
+        }
+        ts.put(e, x);
+        ts.parent[e] = Store::kNone;
+    }
+    // nodes: the one of each split between neighbouring entities, if its leaves are of this
+    // tile and of one segment
+    for (uint32_t k = t; k < uint32_t(C); k += T) {
+        ts.id[k] = kEmpty;
+        ts.parent[C + k] = Store::kNone;
+    }
+    __syncthreads();
+    for (uint32_t k = t; k + 1u < ne; k += T) {
+        const uint32_t q = a.split_node[lastpos[k]];
+        const uint32_t f = a.first[q], l = a.last[q];
+        if (f >= base && l < end && (a.keys[f] >> a.seg_shift) == (a.keys[l] >> a.seg_shift)) ts.id[k] = q;
+    }
+    __syncthreads();
+    for (uint32_t k = t; k + 1u < ne; k += T) {
+        const uint32_t q = ts.id[k];
+        if (q == kEmpty) continue;
+        // a child is the entity beside the split, or the node of a split found by its leaf
+        // (the emitted tree's left child is numbered by the last leaf before the split)
+        uint32_t c[2] = {a.left[q], a.right[q]};
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const uint32_t beside = k + uint32_t(j);
+            if (ts.ref[beside] == c[j]) {
+                c[j] = beside;
             } else {
-                ref[c] = inner[next++];
-                st_set[sp] = sub[c];
-                st_node[sp++] = ref[c];
+                const uint32_t split = a.left[c[j]] & ~kLeafBit;
+                uint32_t lo = 0, hi = ne - 1u;  // the entity that ends at leaf `split`
+                while (lo < hi) {
+                    const uint32_t mid = (lo + hi) >> 1;
+                    if (lastpos[mid] < split) lo = mid + 1u;
+                    else hi = mid;
+                }
+                c[j] = uint32_t(C) + lo;
             }
-            treelet_set_parent(a, ref[c], X);
+            ts.parent[c[j]] = uint16_t(C + k);
         }
-        a.left[X] = ref[0];
-        a.right[X] = ref[1];
+        ts.child[0][k] = uint16_t(c[0]);
+        ts.child[1][k] = uint16_t(c[1]);
     }
-    // children before parents: boxes, costs and counts of the rebuilt nodes
-    uint32_t cnt;
-    for (int k = no - 1; k >= 0; k--) (void)treelet_refresh(a, order[k], &cnt);
-}
-
-__global__ void k_treelets(TreeletArgs a, int n) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    const uint32_t s = find_segment(a.seg_start, a.nseg, uint32_t(p));
-    if (a.seg_start[s + 1] - a.seg_start[s] < 2u) return;  // a one-primitive segment: its parent is above the roots
-    uint32_t node = a.parent_leaf[p];
-    // the walk ends at a segment root; the bound only guards against a broken tree
-    for (int up = 0; node != kEmpty && up < kMaxWalk; up++) {
-        // as in k_fit: the second child to arrive handles the node, and acq_rel makes
-        // everything written below it visible
-        const uint32_t prev = __hip_atomic_fetch_add(&a.visits[node], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (prev == 0u) return;
-        uint32_t count;
-        const float cur = treelet_refresh(a, node, &count);
-        if (count >= 3u) treelet_optimize(a, node, cur);
-        if (a.is_root[node]) return;
-        node = a.parent_int[node];
+    __syncthreads();
+    auto clear_seen = [&]() {
+        if (t < uint32_t(C) / 32u) ts.seen[t] = 0u;
+        __syncthreads();
+    };
+    // the treelet passes, or one pass that only fits the boxes
+    for (uint32_t pass = 0; pass == 0u || pass < a.passes; pass++) {
+        clear_seen();
+        for (uint32_t e0 = t; e0 < ne; e0 += T) {
+            for (uint32_t e = ts.parent[e0]; e != Store::kNone; e = ts.parent[e]) {
+                if (!ts.second(e)) break;
+                uint32_t count;
+                const float cur = tree_refresh(ts, e, count);
+                if (pass < a.passes && count >= 3u) treelet_optimize(ts, e, cur);
+            }
+        }
+        __syncthreads();
+    }
+    if (a.sah) {
+        clear_seen();
+        for (uint32_t e0 = t; e0 < ne; e0 += T) {
+            for (uint32_t e = ts.parent[e0]; e != Store::kNone; e = ts.parent[e]) {
+                if (!ts.second(e)) break;
+                const uint32_t k = e - C;
+                float4 c[2];
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const uint32_t r = ts.child[j][k];
+                    const uint32_t g = ts.is_leaf(r) ? ts.ref[r] : ts.id[r - C];
+                    if (g & kLeafBit) {
+                        const TreeRef x = ts.get(r);
+                        c[j] = sah_leaf(x.l, x.h);
+                    } else {
+                        c[j] = a.cost[g];
+                    }
+                }
+                const TreeRef x = ts.get(e);
+                uint32_t d;
+                const uint32_t q = ts.id[k];
+                a.cost[q] = sah_costs(c[0], c[1], half_area(x.l, x.h), x.n, a.leaf_max, d);
+                a.dec[q] = d;
+            }
+        }
+    }
+    // back to global memory, and the subtrees without a parent here, in leaf order
+    auto global_ref = [&](uint32_t e) { return e < uint32_t(C) ? ts.ref[e] : ts.id[e - C]; };
+    for (uint32_t e = t; e < ne; e += T) {
+        if (ts.parent[e] != Store::kNone) {
+            const uint32_t r = ts.ref[e], q = ts.id[ts.parent[e] - C];
+            if (r & kLeafBit) a.parent_leaf[r & ~kLeafBit] = q;
+            else a.parent_int[r] = q;
+        }
+        const uint32_t q = ts.id[e];
+        if (q == kEmpty) continue;
+        const uint32_t x = C + e;
+        a.left[q] = global_ref(ts.child[0][e]);
+        a.right[q] = global_ref(ts.child[1][e]);
+        if (ts.parent[x] != Store::kNone) a.parent_int[q] = ts.id[ts.parent[x] - C];
+        a.nlo[q] = make_float4(ts.lo[0][x], ts.lo[1][x], ts.lo[2][x], ts.cost[x]);
+        a.nhi[q] = make_float4(ts.hi[0][x], ts.hi[1][x], ts.hi[2][x], 0.f);
+        a.cnt[q] = ts.cnt[x];
+    }
+    if (!roots_out) return;
+    __syncthreads();
+    // the root that starts at each entity: itself, or the topmost node it is the first
+    // entity of (found from the node: its first leaf as emitted, which a root keeps); none
+    // for a finished segment
+    uint32_t* const start = reinterpret_cast<uint32_t*>(ts.lo);  // the boxes are stored
+    auto first_leaf = [&](uint32_t r) { return (r & kLeafBit) ? (r & ~kLeafBit) : a.first[r]; };
+    auto unfinished = [&](uint32_t r) {
+        const uint32_t f = first_leaf(r), l = (r & kLeafBit) ? f : a.last[r];
+        const uint32_t seg = uint32_t(a.keys[f] >> a.seg_shift);
+        return a.seg_start[seg] != f || a.seg_start[seg + 1u] != l + 1u;
+    };
+    for (uint32_t e = t; e < ne; e += T)
+        start[e] = ts.parent[e] == Store::kNone && unfinished(ts.ref[e]) ? ts.ref[e] : kEmpty;
+    __syncthreads();
+    for (uint32_t k = t; k + 1u < ne; k += T) {
+        if (ts.id[k] == kEmpty || ts.parent[C + k] != Store::kNone || !unfinished(ts.id[k])) continue;
+        const uint32_t f = a.first[ts.id[k]];
+        uint32_t lo = 0, hi = ne - 1u;  // the entity that starts at leaf f
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (first_leaf(ts.ref[mid]) < f) lo = mid + 1u;
+            else hi = mid;
+        }
+        start[lo] = ts.id[k];
+    }
+    __syncthreads();
+    uint32_t done = 0;
+    for (uint32_t row = 0; row < ne; row += T) {
+        const uint32_t r = row + t < ne ? start[row + t] : kEmpty;
+        uint32_t total;
+        const uint32_t at = done + block_exclusive<T>(r != kEmpty ? 1u : 0u, s_wave, total);
+        if (r != kEmpty && at < kTileRoots) roots_out[blockIdx.x * kTileRoots + at] = r;
+        done += total;
+    }
+    if (t == 0) {
+        if (done > kTileRoots) atomicOr(a.overflow, kOverflowRoots);  // cannot happen (kTileRoots)
+        count_out[blockIdx.x] = min(done, kTileRoots);
     }
 }
 
@@ -771,7 +1075,9 @@ __global__ void k_treelets(TreeletArgs a, int n) {
 // node below a segment root: the root keeps its run, a right child starts after its
 // left sibling's primitives.  Nodes above the roots are left as built.
 __global__ void k_renumber_nodes(const uint32_t* left, const uint32_t* right, const uint32_t* parent_int,
-                                 const uint32_t* is_root, const uint32_t* cnt, uint32_t* first, uint32_t* last, int ni) {
+                                 const uint32_t* is_root, const uint32_t* cnt, uint32_t* first, uint32_t* last, int ni,
+                                 const uint32_t* overflow) {
+    if (*overflow) return;  // the tree is not complete
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= ni) return;
     uint32_t off = 0, c = uint32_t(i);
@@ -792,7 +1098,9 @@ __global__ void k_renumber_nodes(const uint32_t* left, const uint32_t* right, co
 // new sorted position of each primitive
 __global__ void k_renumber_leaves(const uint32_t* left, const uint32_t* parent_leaf, const uint32_t* first,
                                   const uint32_t* cnt, const uint32_t* seg_start, uint32_t nseg, uint32_t* newpos,
-                                  uint32_t n) {
+                                  uint32_t n,
+                                  const uint32_t* overflow) {
+    if (*overflow) return;  // the tree is not complete
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
     const uint32_t s = find_segment(seg_start, nseg, p);
@@ -805,21 +1113,17 @@ __global__ void k_renumber_leaves(const uint32_t* left, const uint32_t* parent_l
     newpos[p] = first[q] + (l == (kLeafBit | p) ? 0u : ((l & kLeafBit) ? 1u : cnt[l]));
 }
 
-__global__ void k_renumber_apply(const uint32_t* newpos, const uint32_t* perm_in, const uint32_t* pleaf_in,
-                                 uint32_t* perm_out, uint32_t* pleaf_out, uint32_t n) {
+__global__ void k_renumber_apply(const uint32_t* newpos, const uint32_t* perm_in, uint32_t* perm_out, uint32_t* left,
+                                 uint32_t* right, uint32_t n,
+                                 const uint32_t* overflow) {
+    if (*overflow) return;  // the tree is not complete
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
-    const uint32_t q = newpos[p];
-    perm_out[q] = perm_in[p];
-    pleaf_out[q] = pleaf_in[p];
-}
-
-__global__ void k_renumber_refs(uint32_t* left, uint32_t* right, const uint32_t* newpos, int ni) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ni) return;
-    const uint32_t l = left[i], r = right[i];
-    if (l & kLeafBit) left[i] = kLeafBit | newpos[l & ~kLeafBit];
-    if (r & kLeafBit) right[i] = kLeafBit | newpos[r & ~kLeafBit];
+    perm_out[newpos[p]] = perm_in[p];
+    if (p + 1u >= n) return;
+    const uint32_t l = left[p], r = right[p];
+    if (l & kLeafBit) left[p] = kLeafBit | newpos[l & ~kLeafBit];
+    if (r & kLeafBit) right[p] = kLeafBit | newpos[r & ~kLeafBit];
 }
 
 // -------------------------------------------------------------- collapse
@@ -837,11 +1141,12 @@ struct CollapseArgs {
     uint32_t nseg;
     const float* seg_pad;  // absolute padding per segment
     uint32_t leaf_max;
-    WideNode* nodes;
-    uint32_t* node_counter;
+    QNode* nodes;
     uint32_t max_nodes;     // capacity of nodes and of each task array
     uint32_t* overflow;     // set when a capacity would be exceeded
     const uint32_t* dec;    // SAH decision words (NULL: the greedy largest-area collapse)
+    uint2* levels;          // per tree level: tasks, first node of the next level
+    uint32_t* block_sums;   // kCollapseBlocks: internal children of each workgroup's tasks
 };
 
 __device__ inline uint32_t ref_count(const CollapseArgs& a, uint32_t r) {
@@ -850,10 +1155,14 @@ __device__ inline uint32_t ref_count(const CollapseArgs& a, uint32_t r) {
 __device__ inline uint32_t ref_first(const CollapseArgs& a, uint32_t r) {
     return (r & kLeafBit) ? (r & ~kLeafBit) : a.first[r];
 }
-// Collapse of one level, in two passes so node numbering is deterministic:
-// gather picks the (up to 4) children of every task and counts the ones that become
-// internal wide nodes; after an exclusive scan of the counts, emit writes the nodes
-// and numbers the new internal nodes level by level in task order.
+// Collapse of one level, in two launches so node numbering is deterministic: gather
+// picks the (up to 4) children of every task and numbers the ones that become internal
+// wide nodes within its workgroup; emit adds the counts of the workgroups before its own,
+// writes the nodes, quantised, and numbers the new internal nodes level by level in task
+// order.  Level sizes stay on the device, so the host enqueues the levels without
+// waiting for each: a read-back leaves the device idle for 30 to 45 us, a level of 5,000
+// primitives takes 12 us.
+constexpr uint32_t kCollapseBlocks = 1024;
 // task = (binary ref or kEmpty, wide node index, segment)
 // SAH collapse: the children of the wide node made from binary node b, following
 // the decisions (each (ref, slots) pair is expanded until it takes one slot).
@@ -914,87 +1223,105 @@ __device__ inline bool becomes_internal(const CollapseArgs& a, uint32_t r) {
     return ref_count(a, r) > a.leaf_max;
 }
 
-__global__ void k_collapse_gather(CollapseArgs a, const uint4* tasks, uint32_t n, uint4* refs, uint32_t* counts,
-                                  uint32_t* offsets) {
-    uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    uint32_t c[4] = {kEmpty, kEmpty, kEmpty, kEmpty};
-    float3 cl[4], ch[4];
-    int nc = gather_children(a, tasks[t].x, c, cl, ch);
-    uint32_t internal = 0;
-    for (int k = 0; k < nc; k++) internal += becomes_internal(a, c[k]) ? 1u : 0u;
-    refs[t] = make_uint4(c[0], c[1], c[2], c[3]);
-    counts[t] = internal;
-    offsets[t] = internal;
+// tasks of workgroup b of a level with n tasks: whole rows of kBlock
+__device__ inline uint2 collapse_range(uint32_t n) {
+    const uint32_t rows = (n + kBlock - 1) / kBlock, per = (rows + gridDim.x - 1) / gridDim.x;
+    const uint32_t b = min(blockIdx.x * per * kBlock, n);
+    return make_uint2(b, min(b + per * kBlock, n));
 }
 
-__global__ void k_collapse_emit(CollapseArgs a, const uint4* tasks, uint32_t n, const uint4* refs,
-                                const uint32_t* offsets, uint32_t node_base, uint4* tasks_out) {
-    uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    uint4 task = tasks[t];
-    uint32_t w = task.y, seg = task.z;
-    uint4 r4 = refs[t];
-    uint32_t c[4] = {r4.x, r4.y, r4.z, r4.w};
-    float pad = a.seg_pad[seg];
-    uint32_t next = offsets[t];
-    WideNode out;
-    for (int k = 0; k < 4; k++) {
-        if (c[k] == kEmpty) {
-            out.lo_x[k] = out.lo_y[k] = out.lo_z[k] = 0.f;
-            out.hi_x[k] = out.hi_y[k] = out.hi_z[k] = 0.f;
-            out.child[k] = kEmpty;
-            out.count[k] = 0;
-            continue;
+__global__ __launch_bounds__(kBlock) void k_collapse_gather(CollapseArgs a, uint32_t level, const uint4* tasks,
+                                                             uint4* refs, uint32_t* offsets) {
+    __shared__ uint32_t s_wave[kBlock / 64];
+    // (a tree that is not complete has no levels)
+    const uint2 r = collapse_range(*a.overflow ? 0u : a.levels[level].x);
+    uint32_t sum = 0;
+    for (uint32_t row = r.x; row < r.y; row += kBlock) {
+        const uint32_t t = row + threadIdx.x;
+        uint32_t internal = 0;
+        if (t < r.y) {
+            uint32_t c[4] = {kEmpty, kEmpty, kEmpty, kEmpty};
+            float3 cl[4], ch[4];
+            const int nc = gather_children(a, tasks[t].x, c, cl, ch);
+            for (int k = 0; k < nc; k++) internal += becomes_internal(a, c[k]) ? 1u : 0u;
+            refs[t] = make_uint4(c[0], c[1], c[2], c[3]);
         }
-        float3 cl, ch;
-        load_box(c[k], a.lo, a.hi, a.perm, a.nlo, a.nhi, cl, ch);
-        out.lo_x[k] = cl.x - pad; out.lo_y[k] = cl.y - pad; out.lo_z[k] = cl.z - pad;
-        out.hi_x[k] = ch.x + pad; out.hi_y[k] = ch.y + pad; out.hi_z[k] = ch.z + pad;
-        if (!becomes_internal(a, c[k])) {
-            out.child[k] = ref_first(a, c[k]);
-            out.count[k] = ref_count(a, c[k]);
-        } else {
-            uint32_t idx = node_base + next;
-            if (idx >= a.max_nodes || next >= a.max_nodes) {
-                atomicOr(a.overflow, 1u);
+        uint32_t total;
+        const uint32_t off = block_exclusive<kBlock>(internal, s_wave, total);
+        if (t < r.y) offsets[t] = sum + off;
+        sum += total;
+    }
+    if (threadIdx.x == 0) a.block_sums[blockIdx.x] = sum;
+}
+
+__global__ __launch_bounds__(kBlock) void k_collapse_emit(CollapseArgs a, uint32_t level, const uint4* tasks,
+                                                           const uint4* refs, const uint32_t* offsets, uint4* tasks_out) {
+    __shared__ uint32_t s_wave[kBlock / 64];
+    const uint2 lv = a.levels[level];
+    const uint2 r = collapse_range(*a.overflow ? 0u : lv.x);
+    uint32_t mine = 0, before;
+    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kBlock) mine += a.block_sums[b];
+    (void)block_exclusive<kBlock>(mine, s_wave, before);
+    if (blockIdx.x + 1u == gridDim.x && threadIdx.x == 0) {
+        const uint32_t count = before + a.block_sums[blockIdx.x];
+        a.levels[level + 1u] = make_uint2(count, lv.y + count);
+    }
+    for (uint32_t t = r.x + threadIdx.x; t < r.y; t += kBlock) {
+        const uint4 task = tasks[t], r4 = refs[t];
+        const uint32_t seg = task.z;
+        const uint32_t c[4] = {r4.x, r4.y, r4.z, r4.w};
+        const float pad = a.seg_pad[seg];
+        uint32_t next = before + offsets[t];
+        WideNode out;
+        for (int k = 0; k < 4; k++) {
+            if (c[k] == kEmpty) {
+                out.lo_x[k] = out.lo_y[k] = out.lo_z[k] = 0.f;
+                out.hi_x[k] = out.hi_y[k] = out.hi_z[k] = 0.f;
                 out.child[k] = kEmpty;
                 out.count[k] = 0;
                 continue;
             }
-            tasks_out[next] = make_uint4(c[k], idx, seg, 0u);
-            out.child[k] = idx;
-            out.count[k] = 0;
-            next++;
+            float3 cl, ch;
+            load_box(c[k], a.lo, a.hi, a.perm, a.nlo, a.nhi, cl, ch);
+            out.lo_x[k] = cl.x - pad; out.lo_y[k] = cl.y - pad; out.lo_z[k] = cl.z - pad;
+            out.hi_x[k] = ch.x + pad; out.hi_y[k] = ch.y + pad; out.hi_z[k] = ch.z + pad;
+            if (!becomes_internal(a, c[k])) {
+                out.child[k] = ref_first(a, c[k]);
+                out.count[k] = ref_count(a, c[k]);
+            } else {
+                const uint32_t idx = lv.y + next;
+                if (idx >= a.max_nodes || next >= a.max_nodes) {
+                    atomicOr(a.overflow, kOverflowNodes);
+                    out.child[k] = kEmpty;
+                    out.count[k] = 0;
+                    continue;
+                }
+                tasks_out[next] = make_uint4(c[k], idx, seg, 0u);
+                out.child[k] = idx;
+                out.count[k] = 0;
+                next++;
+            }
         }
+        if (task.y < a.max_nodes) a.nodes[task.y] = quantize_node(out);
     }
-    a.nodes[w] = out;
-}
-
-__global__ void k_empty_nodes(WideNode* nodes, uint32_t n) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    WideNode out;
-    for (int k = 0; k < 4; k++) {
-        out.lo_x[k] = out.lo_y[k] = out.lo_z[k] = 0.f;
-        out.hi_x[k] = out.hi_y[k] = out.hi_z[k] = 0.f;
-        out.child[k] = kEmpty;
-        out.count[k] = 0;
-    }
-    nodes[i] = out;
 }
 
 // level 0: one task per segment, its root is node s (kEmpty for an empty segment)
-__global__ void k_init_tasks(const uint32_t* seg_root, uint32_t nseg, uint4* tasks) {
+__global__ void k_init_tasks(const uint32_t* seg_root, uint32_t nseg, uint4* tasks, uint2* levels) {
     uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s == 0u) levels[0] = make_uint2(nseg, nseg);
     if (s >= nseg) return;
     tasks[s] = make_uint4(seg_root[s], s, s, 0u);
 }
 
-// padding and root bounds per segment
-__global__ void k_seg_pad(const uint32_t* bounds, uint32_t nseg, float* pad, float* seg_bounds) {
+// padding and root bounds per segment, and the roots of segments without a binary node
+__global__ void k_seg_pad(const uint32_t* bounds, const uint32_t* seg_start, uint32_t nseg, float* pad,
+                          float* seg_bounds, uint32_t* seg_root, uint32_t* overflow) {
     uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s == 0u) *overflow = 0u;
     if (s >= nseg) return;
+    const uint32_t prims = seg_start[s + 1] - seg_start[s];
+    if (prims < 2u) seg_root[s] = prims ? (kLeafBit | seg_start[s]) : kEmpty;
     const uint32_t* b = bounds + 12 * s;
     float m = 0.f;
     float v[6];
@@ -1204,8 +1531,263 @@ int reorder_instances(hipStream_t st, const InstanceRecord* in, const uint32_t* 
     return 0;
 }
 
+// ------------------------------------------------------------ scratch
+ScratchPool::~ScratchPool() {
+    for (void* p : extra) (void)hipFree(p);
+    if (base) (void)hipFree(base);
+}
+
+void ScratchPool::begin(size_t bytes) {
+    used = 0;
+    if (bytes <= cap) return;
+    if (base) (void)hipFree(base);
+    base = nullptr;
+    cap = 0;
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) {
+        base = (char*)p;
+        cap = bytes;
+    } else {
+        (void)hipGetLastError();  // every buffer is tried by itself then
+    }
+}
+
+void* ScratchPool::alloc_bytes(size_t bytes) {
+    bytes = (bytes + 16 + 255) & ~size_t(255);
+    if (used + bytes <= cap) {
+        void* p = base + used;
+        used += bytes;
+        return p;
+    }
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    extra.push_back(p);
+    return p;
+}
+
+void ScratchPool::end() {
+    used = 0;
+    for (void* p : extra) (void)hipFree(p);
+    extra.clear();
+    if (cap > kScratchKeep) {
+        (void)hipFree(base);
+        base = nullptr;
+        cap = 0;
+    }
+}
+
+size_t lbvh_scratch_bytes(uint32_t n, uint32_t nseg) {
+    const size_t hist = 256 * size_t(blocks_for(n, kRsTile));
+    const size_t nodes = size_t(n) + nseg;
+    const size_t roots = (size_t(blocks_for(n, kTile)) * 5 / 4 + 2) * (kTileRoots + 1) * 4;
+    return size_t(n) * (16 + 8 + 24 + 4 + 4 + 32 + 4 + 16 + 4 + 4) + roots + nodes * (64 + 16 * 3 + 4) +
+           hist * 4 + hist / 128 + size_t(nseg) * 96 + (1u << 16);
+}
+
+int lbvh_build(hipStream_t st, const float4* d_lo, const float4* d_hi, uint32_t n, const uint32_t* d_seg_start,
+               const std::vector<uint32_t>& h_seg_start, uint32_t leaf_max, uint32_t collapse, uint32_t treelet_passes,
+               ScratchPool& s, LbvhResult* out, std::string* err) {
+    const uint32_t nseg = uint32_t(h_seg_start.size()) - 1;
+    if (leaf_max < 1 || leaf_max > uint32_t(kMaxLeafPrims)) { *err = "leaf size out of range"; return int(hipErrorInvalidValue); }
+    if (n >= (1u << kLeafCountShift)) { *err = "too many primitives in one build"; return int(hipErrorInvalidValue); }
+    int segbits = 0;
+    while ((1u << segbits) < nseg) segbits++;
+    int bits = (64 - segbits) / 3;
+    if (bits > 21) bits = 21;
+    const int key_bits = 3 * bits + segbits;
+    const uint32_t max_nodes = n + nseg;
+    uint32_t* bounds = s.alloc<uint32_t>(12 * size_t(nseg));
+    float* pad = s.alloc<float>(nseg);
+    uint32_t* seg_root = s.alloc<uint32_t>(nseg);
+    float* seg_bounds = s.alloc<float>(6 * size_t(nseg));
+    QNode* nodes_tmp = s.alloc<QNode>(max_nodes);
+    constexpr uint32_t kMaxLevels = 256;
+    uint2* levels = s.alloc<uint2>(kMaxLevels + 1);
+    uint32_t* words = s.alloc<uint32_t>(kCollapseBlocks + 1);  // workgroup sums, overflow flag
+    uint4* ta = s.alloc<uint4>(max_nodes);
+    uint4* tb = s.alloc<uint4>(max_nodes);
+    uint4* refs = s.alloc<uint4>(max_nodes);
+    uint32_t* offs = s.alloc<uint32_t>(max_nodes);
+    uint64_t* k0 = s.alloc<uint64_t>(n);
+    uint64_t* k1 = s.alloc<uint64_t>(n);
+    uint32_t* v0 = s.alloc<uint32_t>(n);
+    uint32_t* v1 = s.alloc<uint32_t>(n);
+    uint32_t* left = s.alloc<uint32_t>(n);
+    uint32_t* right = s.alloc<uint32_t>(n);
+    uint32_t* first = s.alloc<uint32_t>(n);
+    uint32_t* last = s.alloc<uint32_t>(n);
+    uint32_t* parent_int = s.alloc<uint32_t>(n);
+    uint32_t* parent_leaf = s.alloc<uint32_t>(n);
+    uint32_t* is_root = s.alloc<uint32_t>(n);
+    uint32_t* split = s.alloc<uint32_t>(n);
+    float4* nlo = s.alloc<float4>(n);
+    float4* nhi = s.alloc<float4>(n);
+    uint32_t* cnt = s.alloc<uint32_t>(n);
+    float4* cost = s.alloc<float4>(n);
+    uint32_t* dec = s.alloc<uint32_t>(n);
+    // the subtrees left by the tiles of a level, ping-pong; sized for the smaller fan, which
+    // has more tiles in every level
+    const size_t tiles0 = blocks_for(n, kTile), tiles1 = (tiles0 + kFanSafe - 1) / kFanSafe;
+    uint32_t* roots0 = s.alloc<uint32_t>(tiles0 * kTileRoots);
+    uint32_t* counts0 = s.alloc<uint32_t>(tiles0);
+    uint32_t* roots1 = s.alloc<uint32_t>(tiles1 * kTileRoots);
+    uint32_t* counts1 = s.alloc<uint32_t>(tiles1);
+    for (const void* p : {(const void*)bounds, (const void*)pad, (const void*)seg_root, (const void*)seg_bounds,
+                          (const void*)nodes_tmp, (const void*)levels, (const void*)words, (const void*)ta, (const void*)tb,
+                          (const void*)refs, (const void*)offs, (const void*)k0, (const void*)k1, (const void*)v0,
+                          (const void*)v1, (const void*)left, (const void*)right, (const void*)first, (const void*)last,
+                          (const void*)parent_int, (const void*)parent_leaf, (const void*)is_root, (const void*)split,
+                          (const void*)nlo, (const void*)nhi, (const void*)cnt, (const void*)cost,
+                          (const void*)dec, (const void*)roots0, (const void*)counts0, (const void*)roots1,
+                          (const void*)counts1})
+        if (!p) { *err = "out of device memory"; return int(hipErrorOutOfMemory); }
+    uint32_t* const overflow = words + kCollapseBlocks;
+    auto fail = [&](int rc, const char* what) {
+        *err = what;
+        return rc;
+    };
+    // launch errors are sticky until read: one check after each group of launches
+    auto launched = [&](const char* what) -> int {
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) *err = what;
+        return int(e);
+    };
+    int rc;
+    hipLaunchKernelGGL(k_init_bounds, dim3(blocks_for(12 * size_t(nseg), kBlock)), dim3(kBlock), 0, st, bounds, nseg);
+    if (n > 0)
+        hipLaunchKernelGGL(k_seg_bounds, dim3(blocks_for(n, bounds_span(n))), dim3(kBlock), 0, st, d_lo, d_hi,
+                           n, d_seg_start, nseg, bounds_span(n), bounds);
+    hipLaunchKernelGGL(k_seg_pad, dim3(blocks_for(nseg, kBlock)), dim3(kBlock), 0, st, bounds, d_seg_start, nseg, pad,
+                       seg_bounds, seg_root, overflow);
+    if ((rc = launched("launch of the segment bounds"))) return rc;
+
+    const uint32_t* perm = v0;
+    const bool sah = collapse == kCollapseSah;
+    if (n > 0) {
+        hipLaunchKernelGGL(k_morton, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, d_lo, d_hi, n, d_seg_start, nseg,
+                           bounds, bits, k0, v0);
+        if (n <= kRankMax) {
+            hipLaunchKernelGGL(k_rank_sort, dim3(blocks_for(n, kRankKeys)), dim3(kRankKeys * kRankSlices), 0, st, k0, v0,
+                               n, k1, v1);
+            std::swap(k0, k1);
+            std::swap(v0, v1);
+            if ((rc = launched("launch k_rank_sort"))) return rc;
+        } else {
+            const uint32_t nblk = blocks_for(n, kRsTile);
+            const uint32_t m = 256u * nblk;
+            uint32_t* hist = s.alloc<uint32_t>(m);
+            const uint32_t scan_cap = 2 * blocks_for(m, kScanPerBlock) + 64;
+            uint32_t* scan_tmp = s.alloc<uint32_t>(scan_cap);
+            if (!hist || !scan_tmp) return fail(int(hipErrorOutOfMemory), "out of device memory");
+            for (int shift = 0; shift < key_bits; shift += 8) {
+                hipLaunchKernelGGL(k_rs_hist, dim3(nblk), dim3(kBlock), 0, st, k0, n, shift, hist, nblk);
+                rc = exclusive_scan(st, hist, m, scan_tmp, scan_cap);
+                if (rc) return fail(rc, "scan");
+                hipLaunchKernelGGL(k_rs_scatter, dim3(nblk), dim3(kBlock), 0, st, k0, v0, k1, v1, n, shift, hist, nblk);
+                std::swap(k0, k1);
+                std::swap(v0, v1);
+            }
+            if ((rc = launched("launch of the radix sort"))) return rc;
+        }
+        // v0: sorted position -> primitive, k0: sorted keys
+    }
+    const uint32_t* const sorted = v0;
+    uint32_t fan = kFan, level = 0, num_nodes = 0, h_over = 0;
+    std::vector<uint2> h_levels(kMaxLevels + 1);
+    for (;; fan = kFanSafe) {
+        if (n > 0) {
+            hipLaunchKernelGGL(k_karras, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, k0, int(n), left, right, first,
+                               last, parent_int, parent_leaf, d_seg_start, nseg, 3 * bits, seg_root, is_root, split);
+            perm = sorted;
+            const TreeArgs tr{d_lo,  d_hi,       sorted,      k0,  3 * bits, d_seg_start, first, last, split,    left, right,
+                              parent_int, parent_leaf, nlo, nhi, cnt,      cost,        dec,   overflow, n, treelet_passes,
+                              leaf_max, sah ? 1u : 0u};
+            uint32_t tiles = blocks_for(n, kTile);
+            uint32_t *ri = roots0, *ci = counts0, *ro = roots1, *co = counts1;
+            hipLaunchKernelGGL((k_tree_level<kTile, kTile, true>), dim3(tiles), dim3(kTile), 0, st, tr, uint32_t(kTile), fan,
+                               (const uint32_t*)nullptr, (const uint32_t*)nullptr, 0u, tiles > 1 ? ri : nullptr, ci);
+            for (uint64_t size = uint64_t(kTile) * fan; tiles > 1; size *= fan) {
+                const uint32_t tiles_in = tiles;
+                tiles = (tiles + fan - 1) / fan;
+                hipLaunchKernelGGL((k_tree_level<kTileRefs, kTileThreads, false>), dim3(tiles), dim3(kTileThreads), 0, st, tr,
+                                   uint32_t(std::min<uint64_t>(size, 1ull << 31)), fan, ri, ci, tiles_in,
+                                   tiles > 1 ? ro : nullptr, co);
+                std::swap(ri, ro);
+                std::swap(ci, co);
+            }
+            if ((rc = launched("launch of the tree passes"))) return rc;
+            if (treelet_passes > 0 && n > 2) {
+                // newpos in offs, which the collapse writes only afterwards
+                hipLaunchKernelGGL(k_renumber_nodes, dim3(blocks_for(n - 1, kBlock)), dim3(kBlock), 0, st, left, right,
+                                   parent_int, is_root, cnt, first, last, int(n) - 1, overflow);
+                hipLaunchKernelGGL(k_renumber_leaves, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, left, parent_leaf,
+                                   first, cnt, d_seg_start, nseg, offs, n, overflow);
+                hipLaunchKernelGGL(k_renumber_apply, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, offs, sorted, v1, left,
+                                   right, n, overflow);
+                perm = v1;
+                if ((rc = launched("launch of the renumbering"))) return rc;
+            }
+        }
+
+        // collapse: level by level until a level has no tasks.  The number of levels is known
+        // on the device only: about 1.25 log4 of the largest segment; more are enqueued when
+        // the levels read back show that the tree goes deeper.
+        CollapseArgs a{d_lo, d_hi, perm, nlo, nhi, left, right, first, last, d_seg_start, nseg, pad, leaf_max,
+                       nodes_tmp, max_nodes, overflow, sah ? dec : nullptr, levels, words};
+        hipLaunchKernelGGL(k_init_tasks, dim3(blocks_for(nseg, kBlock)), dim3(kBlock), 0, st, seg_root, nseg, ta, levels);
+        uint32_t largest = 1;
+        for (uint32_t k = 0; k < nseg; k++) largest = std::max(largest, h_seg_start[k + 1] - h_seg_start[k]);
+        uint32_t want = 1;
+        level = 0;
+        for (uint64_t c = 1; c < largest; c *= 4) want++;
+        want += want / 4;
+        for (bool done = false; !done; want += 4) {
+            for (; level < want && level < kMaxLevels; level++) {
+                const uint64_t bound = std::min<uint64_t>(uint64_t(nseg) << std::min(2u * level, 32u), max_nodes);
+                const dim3 grid(std::min(blocks_for(bound, kBlock), kCollapseBlocks));
+                hipLaunchKernelGGL(k_collapse_gather, grid, dim3(kBlock), 0, st, a, level, ta, refs, offs);
+                hipLaunchKernelGGL(k_collapse_emit, grid, dim3(kBlock), 0, st, a, level, ta, refs, offs, tb);
+                std::swap(ta, tb);
+            }
+            if ((rc = launched("launch of the collapse"))) return rc;
+            if (hipMemcpyAsync(h_levels.data(), levels, sizeof(uint2) * (level + 1), hipMemcpyDeviceToHost, st) != hipSuccess ||
+                hipMemcpyAsync(&h_over, overflow, sizeof(h_over), hipMemcpyDeviceToHost, st) != hipSuccess ||
+                hipStreamSynchronize(st) != hipSuccess)
+                return fail(int(hipErrorUnknown), "read level sizes");
+            if (h_over == kOverflowFan && fan != kFanSafe) break;
+            if (h_over) return fail(int(hipErrorUnknown), "node capacity exceeded during collapse");
+            done = h_levels[level].x == 0u;
+            if (!done && level >= kMaxLevels) return fail(int(hipErrorUnknown), "collapse did not terminate");
+        }
+        if (!h_over) break;
+        // a tile held too many subtrees: once more with tiles that cannot
+        if (hipMemsetAsync(overflow, 0, sizeof(uint32_t), st) != hipSuccess) return fail(int(hipErrorUnknown), "memset");
+    }
+    out->level_start.assign({0u, nseg});
+    num_nodes = nseg;
+    for (uint32_t k = 1; k <= level && h_levels[k].x != 0u; k++) {
+        num_nodes = h_levels[k].y;
+        out->level_start.push_back(num_nodes);
+    }
+    if (num_nodes > max_nodes) return fail(int(hipErrorUnknown), "node capacity exceeded during collapse");
+    QNode* nodes = nullptr;
+    if (hipMalloc(&nodes, sizeof(QNode) * size_t(num_nodes)) != hipSuccess) return fail(int(hipErrorOutOfMemory), "out of device memory");
+    if (hipMemcpyAsync(nodes, nodes_tmp, sizeof(QNode) * size_t(num_nodes), hipMemcpyDeviceToDevice, st) != hipSuccess) {
+        (void)hipFree(nodes);
+        return fail(int(hipErrorUnknown), "copy nodes");
+    }
+    out->nodes = nodes;
+    out->num_nodes = num_nodes;
+    out->perm = perm;
+    out->seg_bounds = seg_bounds;
+    return 0;
+}
+
 namespace {
-// RAII bundle of temporary device buffers.
+// RAII bundle of temporary device buffers (refits).
 struct Scratch {
     std::vector<void*> ptrs;
     ~Scratch() {
@@ -1219,214 +1801,6 @@ struct Scratch {
     }
 };
 }  // namespace
-
-int lbvh_build(hipStream_t st, const float4* d_lo, const float4* d_hi, uint32_t n, const uint32_t* d_seg_start,
-               const std::vector<uint32_t>& h_seg_start, uint32_t leaf_max, uint32_t collapse, uint32_t treelet_passes,
-               LbvhResult* out, std::string* err) {
-    const uint32_t nseg = uint32_t(h_seg_start.size()) - 1;
-    if (leaf_max < 1 || leaf_max > uint32_t(kMaxLeafPrims)) { *err = "leaf size out of range"; return int(hipErrorInvalidValue); }
-    if (n >= (1u << kLeafCountShift)) { *err = "too many primitives in one build"; return int(hipErrorInvalidValue); }
-    int segbits = 0;
-    while ((1u << segbits) < nseg) segbits++;
-    int bits = (64 - segbits) / 3;
-    if (bits > 21) bits = 21;
-    const int key_bits = 3 * bits + segbits;
-    Scratch s;
-    uint32_t* bounds = s.alloc<uint32_t>(12 * size_t(nseg));
-    float* pad = s.alloc<float>(nseg);
-    uint32_t* seg_root = s.alloc<uint32_t>(nseg);
-    const uint32_t max_nodes = n + nseg;
-    WideNode* nodes_tmp = s.alloc<WideNode>(max_nodes);
-    if (!bounds || !pad || !seg_root || !nodes_tmp) { *err = "out of device memory"; return int(hipErrorOutOfMemory); }
-    float* seg_bounds = nullptr;
-    uint32_t* perm_out = nullptr;
-    if (hipMalloc(&seg_bounds, 6 * sizeof(float) * nseg) != hipSuccess) { *err = "out of device memory"; return int(hipErrorOutOfMemory); }
-    if (hipMalloc(&perm_out, sizeof(uint32_t) * (n + 1)) != hipSuccess) {
-        (void)hipFree(seg_bounds);
-        *err = "out of device memory";
-        return int(hipErrorOutOfMemory);
-    }
-    auto fail = [&](int rc, const char* what) {
-        (void)hipFree(seg_bounds);
-        (void)hipFree(perm_out);
-        *err = what;
-        return rc;
-    };
-    int rc;
-    hipLaunchKernelGGL(k_init_bounds, dim3(blocks_for(12 * size_t(nseg), kBlock)), dim3(kBlock), 0, st, bounds, nseg);
-    if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_init_bounds");
-    if (n > 0) {
-        hipLaunchKernelGGL(k_seg_bounds, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, d_lo, d_hi, n, d_seg_start,
-                           nseg, bounds);
-        if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_seg_bounds");
-    }
-    hipLaunchKernelGGL(k_seg_pad, dim3(blocks_for(nseg, kBlock)), dim3(kBlock), 0, st, bounds, nseg, pad, seg_bounds);
-    if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_seg_pad");
-    if (hipMemsetAsync(seg_root, 0xFF, sizeof(uint32_t) * nseg, st) != hipSuccess) return fail(int(hipErrorUnknown), "memset");
-
-    uint32_t* nc = s.alloc<uint32_t>(4);  // node counter, task counters
-    if (!nc) return fail(int(hipErrorOutOfMemory), "out of device memory");
-    if (n > 0) {
-        uint64_t* k0 = s.alloc<uint64_t>(n);
-        uint64_t* k1 = s.alloc<uint64_t>(n);
-        uint32_t* v0 = s.alloc<uint32_t>(n);
-        uint32_t* v1 = s.alloc<uint32_t>(n);
-        const uint32_t nblk = blocks_for(n, kRsTile);
-        const uint32_t m = 256u * nblk;
-        uint32_t* hist = s.alloc<uint32_t>(m);
-        const uint32_t scan_cap = 2 * blocks_for(m, kScanPerBlock) + 64;
-        uint32_t* scan_tmp = s.alloc<uint32_t>(scan_cap);
-        if (!k0 || !k1 || !v0 || !v1 || !hist || !scan_tmp) return fail(int(hipErrorOutOfMemory), "out of device memory");
-        hipLaunchKernelGGL(k_morton, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, d_lo, d_hi, n, d_seg_start, nseg,
-                           bounds, bits, k0, v0);
-        if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_morton");
-        for (int shift = 0; shift < key_bits; shift += 8) {
-            hipLaunchKernelGGL(k_rs_hist, dim3(nblk), dim3(kBlock), 0, st, k0, n, shift, hist, nblk);
-            if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_rs_hist");
-            rc = exclusive_scan(st, hist, m, scan_tmp, scan_cap);
-            if (rc) return fail(rc, "scan");
-            hipLaunchKernelGGL(k_rs_scatter, dim3(nblk), dim3(kBlock), 0, st, k0, v0, k1, v1, n, shift, hist, nblk);
-            if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_rs_scatter");
-            std::swap(k0, k1);
-            std::swap(v0, v1);
-        }
-        // v0 = perm (sorted position -> primitive), k0 = sorted keys
-        if (hipMemcpyAsync(perm_out, v0, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st) != hipSuccess)
-            return fail(int(hipErrorUnknown), "copy perm");
-        const int ni = int(n) - 1;
-        uint32_t* left = s.alloc<uint32_t>(n);
-        uint32_t* right = s.alloc<uint32_t>(n);
-        uint32_t* first = s.alloc<uint32_t>(n);
-        uint32_t* last = s.alloc<uint32_t>(n);
-        uint32_t* parent_int = s.alloc<uint32_t>(n);
-        uint32_t* parent_leaf = s.alloc<uint32_t>(n);
-        uint32_t* is_root = s.alloc<uint32_t>(n);
-        uint32_t* visits = s.alloc<uint32_t>(n);
-        float4* nlo = s.alloc<float4>(n);
-        float4* nhi = s.alloc<float4>(n);
-        if (!left || !right || !first || !last || !parent_int || !parent_leaf || !is_root || !visits || !nlo || !nhi)
-            return fail(int(hipErrorOutOfMemory), "out of device memory");
-        if (hipMemsetAsync(parent_int, 0xFF, sizeof(uint32_t) * n, st) != hipSuccess ||
-            hipMemsetAsync(parent_leaf, 0xFF, sizeof(uint32_t) * n, st) != hipSuccess ||
-            hipMemsetAsync(is_root, 0, sizeof(uint32_t) * n, st) != hipSuccess ||
-            hipMemsetAsync(visits, 0, sizeof(uint32_t) * n, st) != hipSuccess)
-            return fail(int(hipErrorUnknown), "memset");
-        if (ni > 0) {
-            hipLaunchKernelGGL(k_karras, dim3(blocks_for(ni, kBlock)), dim3(kBlock), 0, st, k0, int(n), left, right,
-                               first, last, parent_int, parent_leaf, d_seg_start, nseg, 3 * bits, seg_root);
-            if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_karras");
-        }
-        hipLaunchKernelGGL(k_single_roots, dim3(blocks_for(nseg, kBlock)), dim3(kBlock), 0, st, d_seg_start, nseg,
-                           seg_root);
-        hipLaunchKernelGGL(k_mark_roots, dim3(blocks_for(nseg, kBlock)), dim3(kBlock), 0, st, seg_root, nseg, is_root);
-        // sorted position -> primitive, and each primitive's parent (both renumbered
-        // by the treelet passes)
-        const uint32_t* perm = v0;
-        const uint32_t* pleaf = parent_leaf;
-        if (treelet_passes > 0 && ni >= 2) {
-            uint32_t* cnt = s.alloc<uint32_t>(n);
-            uint32_t* newpos = s.alloc<uint32_t>(n);
-            uint32_t* pleaf2 = s.alloc<uint32_t>(n);
-            if (!cnt || !newpos || !pleaf2) return fail(int(hipErrorOutOfMemory), "out of device memory");
-            TreeletArgs ta{d_lo, d_hi, v0, left, right, parent_int, parent_leaf, is_root, visits, nlo, nhi, cnt,
-                           d_seg_start, nseg};
-            for (uint32_t pass = 0; pass < treelet_passes; pass++) {
-                if (hipMemsetAsync(visits, 0, sizeof(uint32_t) * n, st) != hipSuccess) return fail(int(hipErrorUnknown), "memset");
-                hipLaunchKernelGGL(k_treelets, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, ta, int(n));
-                if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_treelets");
-            }
-            hipLaunchKernelGGL(k_renumber_nodes, dim3(blocks_for(ni, kBlock)), dim3(kBlock), 0, st, left, right,
-                               parent_int, is_root, cnt, first, last, ni);
-            hipLaunchKernelGGL(k_renumber_leaves, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, left, parent_leaf,
-                               first, cnt, d_seg_start, nseg, newpos, n);
-            hipLaunchKernelGGL(k_renumber_apply, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, newpos, v0,
-                               parent_leaf, perm_out, pleaf2, n);
-            hipLaunchKernelGGL(k_renumber_refs, dim3(blocks_for(ni, kBlock)), dim3(kBlock), 0, st, left, right, newpos, ni);
-            if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch renumbering");
-            if (hipMemsetAsync(visits, 0, sizeof(uint32_t) * n, st) != hipSuccess) return fail(int(hipErrorUnknown), "memset");
-            perm = perm_out;
-            pleaf = pleaf2;
-        }
-        const bool sah = collapse == kCollapseSah;
-        SahArgs sa{nullptr, nullptr, first, last, leaf_max};
-        if (sah) {
-            sa.cost = s.alloc<float4>(n);
-            sa.dec = s.alloc<uint32_t>(n);
-            if (!sa.cost || !sa.dec) return fail(int(hipErrorOutOfMemory), "out of device memory");
-            hipLaunchKernelGGL(k_fit<true>, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, d_lo, d_hi, perm, int(n),
-                               left, right, parent_int, pleaf, is_root, visits, nlo, nhi, sa);
-        } else {
-            hipLaunchKernelGGL(k_fit<false>, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, d_lo, d_hi, perm, int(n),
-                               left, right, parent_int, pleaf, is_root, visits, nlo, nhi, sa);
-        }
-        if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_fit");
-
-        CollapseArgs a{d_lo, d_hi, perm, nlo, nhi, left, right, first, last, d_seg_start, nseg, pad, leaf_max,
-                       nodes_tmp, nc, max_nodes, nc + 3, sa.dec};
-        uint4* ta = s.alloc<uint4>(max_nodes);
-        uint4* tb = s.alloc<uint4>(max_nodes);
-        uint4* refs = s.alloc<uint4>(max_nodes);
-        uint32_t* counts = s.alloc<uint32_t>(max_nodes);
-        uint32_t* offs = s.alloc<uint32_t>(max_nodes);
-        const uint32_t ccap = 2 * blocks_for(max_nodes, kScanPerBlock) + 64;
-        uint32_t* ctmp = s.alloc<uint32_t>(ccap);
-        if (!ta || !tb || !refs || !counts || !offs || !ctmp) return fail(int(hipErrorOutOfMemory), "out of device memory");
-        if (hipMemsetAsync(nc, 0, 4 * sizeof(uint32_t), st) != hipSuccess) return fail(int(hipErrorUnknown), "memset");
-        hipLaunchKernelGGL(k_init_tasks, dim3(blocks_for(nseg, kBlock)), dim3(kBlock), 0, st, seg_root, nseg, ta);
-        if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_init_tasks");
-        uint32_t count = nseg, node_base = nseg;
-        out->level_start.assign({0u, nseg});
-        for (int level = 0; count > 0; level++) {
-            if (level > 200) return fail(int(hipErrorUnknown), "collapse did not terminate");
-            hipLaunchKernelGGL(k_collapse_gather, dim3(blocks_for(count, kBlock)), dim3(kBlock), 0, st, a, ta, count,
-                               refs, counts, offs);
-            if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_collapse_gather");
-            rc = exclusive_scan(st, offs, count, ctmp, ccap);
-            if (rc) return fail(rc, "scan");
-            hipLaunchKernelGGL(k_collapse_emit, dim3(blocks_for(count, kBlock)), dim3(kBlock), 0, st, a, ta, count,
-                               refs, offs, node_base, tb);
-            if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_collapse_emit");
-            uint32_t last[2] = {0, 0};
-            if (hipMemcpyAsync(&last[0], offs + count - 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st) != hipSuccess ||
-                hipMemcpyAsync(&last[1], counts + count - 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st) != hipSuccess ||
-                hipStreamSynchronize(st) != hipSuccess)
-                return fail(int(hipErrorUnknown), "read level size");
-            count = last[0] + last[1];
-            node_base += count;
-            if (count) out->level_start.push_back(node_base);
-            if (node_base > max_nodes) return fail(int(hipErrorUnknown), "node capacity exceeded during collapse");
-            std::swap(ta, tb);
-        }
-        if (hipMemcpyAsync(nc, &node_base, sizeof(uint32_t), hipMemcpyHostToDevice, st) != hipSuccess)
-            return fail(int(hipErrorUnknown), "copy node count");
-    } else {
-        // no primitives at all: every segment root is an empty node
-        out->level_start.assign({0u, nseg});
-        uint32_t h_init[4] = {nseg, 0, 0, 0};
-        if (hipMemcpyAsync(nc, h_init, sizeof(h_init), hipMemcpyHostToDevice, st) != hipSuccess)
-            return fail(int(hipErrorUnknown), "copy counters");
-        hipLaunchKernelGGL(k_empty_nodes, dim3(blocks_for(nseg, kBlock)), dim3(kBlock), 0, st, nodes_tmp, nseg);
-        if (hipGetLastError() != hipSuccess) return fail(int(hipErrorLaunchFailure), "launch k_empty_nodes");
-    }
-    uint32_t hc[4] = {0, 0, 0, 0};
-    if (hipMemcpyAsync(hc, nc, sizeof(hc), hipMemcpyDeviceToHost, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
-        return fail(int(hipErrorUnknown), "read node count");
-    if (hc[3] != 0u || hc[0] > max_nodes) return fail(int(hipErrorUnknown), "node capacity exceeded during collapse");
-    uint32_t num_nodes = hc[0];
-    QNode* nodes = nullptr;
-    if (hipMalloc(&nodes, sizeof(QNode) * size_t(num_nodes)) != hipSuccess) return fail(int(hipErrorOutOfMemory), "out of device memory");
-    hipLaunchKernelGGL(k_quantize_nodes, dim3(blocks_for(num_nodes, kBlock)), dim3(kBlock), 0, st,
-                       (const WideNode*)nodes_tmp, num_nodes, nodes);
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) {
-        (void)hipFree(nodes);
-        return fail(int(hipErrorUnknown), "quantise nodes");
-    }
-    out->nodes = nodes;
-    out->num_nodes = num_nodes;
-    out->perm = perm_out;
-    out->seg_bounds = seg_bounds;
-    return 0;
-}
 
 int lbvh_refit(hipStream_t st, const TriSegment* d_segs, uint32_t nseg, uint32_t n, float4* d_tri, QNode* d_nodes,
                uint32_t num_nodes, const std::vector<uint32_t>& level_start, BlasDesc* d_descs, uint32_t* d_bad,
