@@ -525,22 +525,22 @@ int rt_refit_blas_batch(rt_ctx* ctx, const rt_blas_input* inputs, uint32_t count
     int rc = make_segments(ctx, inputs, count, segs, seg_start, total);
     if (rc) return rc;
     hipStream_t st = ctx->stream;
-    hipError_t e;
-    DevPtr d_segs(dev_alloc<TriSegment>(count, &e));
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-    DevPtr d_bad(dev_alloc<uint32_t>(1, &e));
-    if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc");
-    RT_HIP(ctx, hipMemcpyAsync(d_segs.get(), segs.data(), sizeof(TriSegment) * count, hipMemcpyHostToDevice, st), "copy segments");
-    RT_HIP(ctx, hipMemsetAsync(d_bad.get(), 0, sizeof(uint32_t), st), "memset");
+    ScratchScope scope(ctx->scratch, refit_scratch_bytes(pool->num_nodes, count, 0) + (sizeof(TriSegment) + 4) * size_t(count));
+    ScratchPool& sc = ctx->scratch;
+    TriSegment* d_segs = sc.alloc<TriSegment>(count);
+    uint32_t* d_bad = sc.alloc<uint32_t>(1);
+    if (!d_segs || !d_bad) return fail(ctx, RT_ERR_OUT_OF_MEMORY, "BLAS refit: out of device memory");
+    RT_HIP(ctx, hipMemcpyAsync(d_segs, segs.data(), sizeof(TriSegment) * count, hipMemcpyHostToDevice, st), "copy segments");
+    RT_HIP(ctx, hipMemsetAsync(d_bad, 0, sizeof(uint32_t), st), "memset");
     std::string err;
-    rc = lbvh_refit(st, (const TriSegment*)d_segs.get(), count, pool->num_tris, (float4*)pool->tris.get(),
-                    (QNode*)pool->nodes.get(), pool->num_nodes, pool->level_start, (BlasDesc*)pool->descs.get(),
-                    (uint32_t*)d_bad.get(), &err);
+    rc = lbvh_refit(st, d_segs, count, pool->num_tris, (float4*)pool->tris.get(), (QNode*)pool->nodes.get(),
+                    pool->num_nodes, pool->level_start, (BlasDesc*)pool->descs.get(), d_bad, sc, &err);
     if (rc) return fail(ctx, rc == int(hipErrorOutOfMemory) ? RT_ERR_OUT_OF_MEMORY : RT_ERR_HIP, "BLAS refit: " + err);
     uint32_t bad = 0;
     std::vector<BlasDesc> descs(count);
-    RT_HIP(ctx, hipMemcpy(&bad, d_bad.get(), sizeof(uint32_t), hipMemcpyDeviceToHost), "copy flag");
-    RT_HIP(ctx, hipMemcpy(descs.data(), pool->descs.get(), sizeof(BlasDesc) * count, hipMemcpyDeviceToHost), "copy descs");
+    RT_HIP(ctx, hipMemcpyAsync(&bad, d_bad, sizeof(uint32_t), hipMemcpyDeviceToHost, st), "copy flag");
+    RT_HIP(ctx, hipMemcpyAsync(descs.data(), pool->descs.get(), sizeof(BlasDesc) * count, hipMemcpyDeviceToHost, st), "copy descs");
+    RT_HIP(ctx, hipStreamSynchronize(st), "hipStreamSynchronize");
     for (uint32_t i = 0; i < count; i++) std::memcpy(ents[i]->h_desc.bounds, descs[i].bounds, sizeof(descs[i].bounds));
     if (bad) return fail(ctx, RT_ERR_INVALID_ARGUMENT, "an index exceeds max_vertex");
     return RT_OK;
@@ -740,15 +740,17 @@ int rt_refit_tlas(rt_ctx* ctx, rt_tlas tlas) {
     DeviceGuard g(ctx->device);
     hipStream_t st = ctx->stream;
     std::string err;
+    ScratchScope scope(ctx->scratch, refit_scratch_bytes(te.flat_num_tris ? te.flat_num_nodes : 0, 1, 0) +
+                                         refit_scratch_bytes(te.num_nodes, 1, te.num_tlas));
     if (te.flat_num_tris) {
         int rc = lbvh_refit_flat(st, (const InstanceRecord*)te.inst.get(), te.flat_num_tris, (float4*)te.flat_tris.get(),
                                  (QNode*)te.flat_nodes.get(), te.flat_num_nodes, te.flat_level_start, te.flat_bounds,
-                                 &err);
+                                 ctx->scratch, &err);
         if (rc) return fail(ctx, rc == int(hipErrorOutOfMemory) ? RT_ERR_OUT_OF_MEMORY : RT_ERR_HIP, "flattened BVH refit: " + err);
     }
     if (te.num_tlas) {
         int rc = lbvh_refit_instances(st, (const InstanceRecord*)te.inst.get(), te.num_tlas, (QNode*)te.nodes.get(),
-                                      te.num_nodes, te.level_start, te.bounds, &err);
+                                      te.num_nodes, te.level_start, te.bounds, ctx->scratch, &err);
         if (rc) return fail(ctx, rc == int(hipErrorOutOfMemory) ? RT_ERR_OUT_OF_MEMORY : RT_ERR_HIP, "TLAS refit: " + err);
     }
     return RT_OK;

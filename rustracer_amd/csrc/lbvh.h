@@ -102,28 +102,33 @@ struct FlatSource {
 int gather_flat(hipStream_t stream, const FlatSource* d_src, uint32_t nsrc, uint32_t n, float4* d_tri, float4* d_lo,
                 float4* d_hi);
 
+// bytes a refit takes from the pool, about: of num_nodes nodes, nseg segments, and
+// `boxes` leaf boxes (instances)
+size_t refit_scratch_bytes(uint32_t num_nodes, uint32_t nseg, uint32_t boxes);
+
 // Refit of a built BLAS pool to new vertex data with the same topology: rewrites the
 // triangle records' positions from `d_segs` (record r keeps its primitive index and
 // segment), then recomputes every node's child boxes bottom-up level by level, padded
 // and quantised as the build does, and the BlasDescs' root bounds.  Sets *d_bad to 1
 // if an index exceeds its segment's max_vertex or a primitive index its segment's
-// count.
+// count.  Enqueues only: the scratch must stay until the stream is done.
 int lbvh_refit(hipStream_t stream, const TriSegment* d_segs, uint32_t nseg, uint32_t n, float4* d_tri, QNode* d_nodes,
                uint32_t num_nodes, const std::vector<uint32_t>& level_start, BlasDesc* d_descs, uint32_t* d_bad,
-               std::string* err);
+               ScratchPool& scratch, std::string* err);
 
 // Refit of a flattened BVH (one segment, root node 0) after the BLASes its records
 // come from were refit: every record takes its positions again from its BLAS record,
 // then the node boxes are recomputed bottom-up as in lbvh_refit.  `bounds` gets the
 // padded root box.
 int lbvh_refit_flat(hipStream_t stream, const InstanceRecord* d_inst, uint32_t n, float4* d_tri, QNode* d_nodes,
-                    uint32_t num_nodes, const std::vector<uint32_t>& level_start, float bounds[6], std::string* err);
+                    uint32_t num_nodes, const std::vector<uint32_t>& level_start, float bounds[6],
+                    ScratchPool& scratch, std::string* err);
 
 // Refit of the TLAS over n instance records in leaf order (their BLAS bounds and
 // transforms as they are now), node boxes recomputed bottom-up.
 int lbvh_refit_instances(hipStream_t stream, const InstanceRecord* d_inst, uint32_t n, QNode* d_nodes,
                          uint32_t num_nodes, const std::vector<uint32_t>& level_start, float bounds[6],
-                         std::string* err);
+                         ScratchPool& scratch, std::string* err);
 
 // Instance boxes (world space) for the TLAS build.
 int prepare_instances(hipStream_t stream, const InstanceRecord* d_inst, uint32_t n, float4* d_lo,

@@ -1340,66 +1340,121 @@ __global__ void k_seg_pad(const uint32_t* bounds, const uint32_t* seg_start, uin
 }
 
 // ------------------------------------------------------------ refit
-// Record r of the pool gets new positions for its primitive (v0.w, kept) of the
-// segment whose records contain r; the other words are kept.  Raises the segment's
-// largest coordinate magnitude (non-negative floats order as their bits).
-__global__ void k_refit_records(const TriSegment* segs, uint32_t nseg, uint32_t n, float4* tri, uint32_t* seg_mag,
-                                uint32_t* bad) {
-    uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n) return;
+// Largest coordinate magnitudes (non-negative floats order as their bits).  The maxima of
+// one segment go to one word, one after another: a wave brings one (when it is of one
+// segment), a workgroup whose whole span is of one segment one.
+__device__ inline uint32_t wave_max(uint32_t v) {
+    for (int o = 32; o > 0; o >>= 1) v = max(v, uint32_t(__shfl_xor(int(v), o, 64)));
+    return v;
+}
+__device__ inline void raise_block(uint32_t* word, uint32_t v) {  // every thread
+    __shared__ uint32_t s_max[kBlock / 64];
+    v = wave_max(v);
+    if ((threadIdx.x & 63u) == 0u) s_max[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x != 0u) return;
+    for (int w = 1; w < kBlock / 64; w++) v = max(v, s_max[w]);
+    atomicMax(word, v);
+}
+__device__ inline void raise_wave(uint32_t* words, uint32_t seg, uint32_t v, bool valid) {  // every lane
+    if (!__ballot(valid)) return;
+    const uint32_t w0 = __shfl(seg, 0, 64);  // lane 0 is valid when any lane is
+    if (__ballot(valid && seg != w0) == 0ull) {
+        v = wave_max(valid ? v : 0u);
+        if (__lane_id() == 0) atomicMax(words + w0, v);
+    } else if (valid) {
+        atomicMax(words + seg, v);
+    }
+}
+__device__ inline uint32_t tri_mag(float3 a, float3 b, float3 c) {
+    const float3 v[3] = {a, b, c};
+    float mag = 0.f;
+    for (int k = 0; k < 3; k++) mag = fmaxf(mag, fmaxf(fabsf(v[k].x), fmaxf(fabsf(v[k].y), fabsf(v[k].z))));
+    return isfinite(mag) ? __float_as_uint(mag) : 0u;
+}
+__device__ inline uint32_t find_tri_segment(const TriSegment* segs, uint32_t nseg, uint32_t r) {
     uint32_t a = 0, b = nseg;
     while (b - a > 1) {
         uint32_t m = (a + b) >> 1;
         if (segs[m].prim_start <= r) a = m; else b = m;
     }
-    const TriSegment& s = segs[a];
-    float4* t = tri + 3 * size_t(r);
-    const float4 t0 = t[0], t1 = t[1], t2 = t[2];
-    const uint32_t prim = __float_as_uint(t0.w);
-    float3 v[3];
-    bool ok = prim < s.prim_count;
-    for (int k = 0; k < 3; k++) {
-        uint32_t idx = ok ? s.index_data[3 * size_t(prim) + k] : 0u;
-        if (idx > s.max_vertex) { ok = false; idx = 0; }
-        const float* f = (const float*)(s.vertex_data + size_t(s.first_vertex + idx) * s.stride);
-        v[k] = mk3(f[0], f[1], f[2]);
-    }
-    if (!ok) {
-        atomicOr(bad, 1u);
-        v[1] = v[0];
-        v[2] = v[0];
-    }
-    t[0] = make_float4(v[0].x, v[0].y, v[0].z, t0.w);
-    t[1] = make_float4(v[1].x, v[1].y, v[1].z, t1.w);
-    t[2] = make_float4(v[2].x, v[2].y, v[2].z, t2.w);
-    float mag = 0.f;
-    for (int k = 0; k < 3; k++) mag = fmaxf(mag, fmaxf(fabsf(v[k].x), fmaxf(fabsf(v[k].y), fabsf(v[k].z))));
-    if (isfinite(mag)) atomicMax(seg_mag + a, __float_as_uint(mag));
+    return a;
 }
 
-// Segment of each node: the roots are nodes 0..nseg-1, and the internal children of
-// one level's nodes inherit their parent's segment (run top-down, level by level).
-__global__ void k_refit_seg(const QNode* nodes, uint32_t begin, uint32_t end, uint32_t* node_seg) {
-    uint32_t i = begin + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= end) return;
-    const QNode q = nodes[i];
-    const uint32_t seg = node_seg[i];
-    for (int k = 0; k < 4; k++)
-        if (q.child[k] != kEmpty && q.count[k] == 0) node_seg[q.child[k]] = seg;
+// Record r of the pool gets new positions for its primitive (v0.w, kept) of the
+// segment whose records contain r; the other words are kept.  Raises the segment's
+// largest coordinate magnitude (200k triangles: 467 us with an atomic per triangle,
+// 13 us with one per span).
+__global__ __launch_bounds__(kBlock) void k_refit_records(const TriSegment* segs, uint32_t nseg, uint32_t n,
+                                                          uint32_t span, float4* tri, uint32_t* seg_mag,
+                                                          uint32_t* bad) {
+    const uint32_t base = blockIdx.x * span, end = base + min(span, n - base);
+    const uint32_t s0 = find_tri_segment(segs, nseg, base);
+    const bool one = s0 == find_tri_segment(segs, nseg, end - 1u);
+    uint32_t most = 0;
+    for (uint32_t row = base; row < end; row += kBlock) {
+        const uint32_t r = row + threadIdx.x;
+        const bool valid = r < end;
+        uint32_t a = s0, mag = 0;
+        if (valid) {
+            if (!one) a = find_tri_segment(segs, nseg, r);
+            const TriSegment& s = segs[a];
+            float4* t = tri + 3 * size_t(r);
+            const float4 t0 = t[0], t1 = t[1], t2 = t[2];
+            const uint32_t prim = __float_as_uint(t0.w);
+            float3 v[3];
+            bool ok = prim < s.prim_count;
+            for (int k = 0; k < 3; k++) {
+                uint32_t idx = ok ? s.index_data[3 * size_t(prim) + k] : 0u;
+                if (idx > s.max_vertex) { ok = false; idx = 0; }
+                const float* f = (const float*)(s.vertex_data + size_t(s.first_vertex + idx) * s.stride);
+                v[k] = mk3(f[0], f[1], f[2]);
+            }
+            if (!ok) {
+                atomicOr(bad, 1u);
+                v[1] = v[0];
+                v[2] = v[0];
+            }
+            t[0] = make_float4(v[0].x, v[0].y, v[0].z, t0.w);
+            t[1] = make_float4(v[1].x, v[1].y, v[1].z, t1.w);
+            t[2] = make_float4(v[2].x, v[2].y, v[2].z, t2.w);
+            mag = tri_mag(v[0], v[1], v[2]);
+        }
+        most = max(most, mag);
+        if (!one) raise_wave(seg_mag, a, mag, valid);
+    }
+    if (one) raise_block(seg_mag + s0, most);
 }
 
-// One level, bottom-up: child boxes from the triangle records (leaves) or from the
-// refit boxes of the deeper level (internal children), padded by the segment's
-// padding as the build pads them, quantised; the node's own (unpadded) box is kept
-// for its parent.
-template <bool kBoxLeaves>
-__global__ void k_refit_level(QNode* nodes, uint32_t begin, uint32_t end, const float4* tri, const float4* leaf_lo,
-                              const float4* leaf_hi, const uint32_t* node_seg, const uint32_t* seg_mag, float* node_box) {
-    uint32_t i = begin + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= end) return;
-    const QNode q = nodes[i];
+// Bottom-up over the levels of a forest: child boxes from the triangle records or boxes
+// (leaves) or from the refit boxes of the deeper level (internal children), padded by the
+// segment's padding as the build pads them, quantised; the node's own (unpadded) box is
+// kept for its parent, and so is its segment, which a leaf child finds by its record.
+// Root bounds (padded, 0 for an empty segment) go to descs, as the build reports them.
+struct RefitArgs {
+    QNode* nodes;
+    uint32_t nseg;           // roots: nodes 0..nseg-1, root s is of segment s
+    const TriSegment* segs;  // NULL: one segment
+    const float4* tri;
+    const float4* leaf_lo;   // boxes in place of triangles (tri NULL)
+    const float4* leaf_hi;
+    const uint32_t* seg_mag;
+    uint32_t* node_seg;
+    float* node_box;
+    BlasDesc* descs;
+};
+
+__device__ inline void refit_node(const RefitArgs& a, uint32_t i) {
+    const QNode q = a.nodes[i];
+    uint32_t seg = i < a.nseg ? i : 0u;
+    if (a.segs && i >= a.nseg) {
+        // (below a root a node has a child)
+        if (q.count[0]) seg = find_tri_segment(a.segs, a.nseg, q.child[0]);
+        else if (q.child[0] != kEmpty) seg = a.node_seg[q.child[0]];
+        a.node_seg[i] = seg;
+    }
     // about 8 ulp of the segment's largest coordinate magnitude (as the build pads)
-    const float pad = __uint_as_float(seg_mag[node_seg[i]]) * 9.5367431640625e-07f + 1e-30f;
+    const float pad = __uint_as_float(a.seg_mag[seg]) * 9.5367431640625e-07f + 1e-30f;
     WideNode w;
     float3 nl = mk3(INFINITY, INFINITY, INFINITY), nh = mk3(-INFINITY, -INFINITY, -INFINITY);
     for (int k = 0; k < 4; k++) {
@@ -1414,12 +1469,12 @@ __global__ void k_refit_level(QNode* nodes, uint32_t begin, uint32_t end, const 
         float3 l = mk3(INFINITY, INFINITY, INFINITY), h = mk3(-INFINITY, -INFINITY, -INFINITY);
         if (cnt) {
             for (uint32_t r = c; r < c + cnt; r++) {
-                if (kBoxLeaves) {
-                    l = fmin3(l, xyz(leaf_lo[r]));
-                    h = fmax3(h, xyz(leaf_hi[r]));
+                if (!a.tri) {
+                    l = fmin3(l, xyz(a.leaf_lo[r]));
+                    h = fmax3(h, xyz(a.leaf_hi[r]));
                     continue;
                 }
-                const float4* t = tri + 3 * size_t(r);
+                const float4* t = a.tri + 3 * size_t(r);
                 for (int v = 0; v < 3; v++) {
                     const float3 p = xyz(t[v]);
                     l = fmin3(l, p);
@@ -1427,7 +1482,7 @@ __global__ void k_refit_level(QNode* nodes, uint32_t begin, uint32_t end, const 
                 }
             }
         } else {
-            const float* b = node_box + 6 * size_t(c);
+            const float* b = a.node_box + 6 * size_t(c);
             l = mk3(b[0], b[1], b[2]);
             h = mk3(b[3], b[4], b[5]);
         }
@@ -1436,59 +1491,71 @@ __global__ void k_refit_level(QNode* nodes, uint32_t begin, uint32_t end, const 
         w.lo_x[k] = l.x - pad; w.lo_y[k] = l.y - pad; w.lo_z[k] = l.z - pad;
         w.hi_x[k] = h.x + pad; w.hi_y[k] = h.y + pad; w.hi_z[k] = h.z + pad;
     }
-    float* b = node_box + 6 * size_t(i);
+    float* b = a.node_box + 6 * size_t(i);
     b[0] = nl.x; b[1] = nl.y; b[2] = nl.z;
     b[3] = nh.x; b[4] = nh.y; b[5] = nh.z;
-    nodes[i] = quantize_node(w);
+    a.nodes[i] = quantize_node(w);
+    if (i < a.nseg) {
+        const bool empty = !(nl.x <= nh.x);
+        const float v[6] = {nl.x - pad, nl.y - pad, nl.z - pad, nh.x + pad, nh.y + pad, nh.z + pad};
+        for (int k = 0; k < 6; k++) a.descs[i].bounds[k] = empty ? 0.f : v[k];
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_refit_level(RefitArgs a, uint32_t begin, uint32_t end) {
+    const uint32_t i = begin + blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < end) refit_node(a, i);
+}
+
+// Consecutive levels of at most kRefitSmall nodes in one workgroup, with a barrier between
+// them.  A level takes about 8 us either way (a chain of loads, then the quantising); what
+// goes is its launch: 627 to 593 us an animation step of 1,300 triangles, no change for
+// 200k, where the large levels set the pace.
+constexpr uint32_t kRefitSmall = 1024;
+constexpr int kRefitLevels = 16, kRefitThreads = 1024;
+struct RefitLevels {
+    uint32_t count;
+    uint32_t start[kRefitLevels + 1];  // ascending: levels are taken from the last to the first
+};
+__global__ __launch_bounds__(kRefitThreads) void k_refit_levels(RefitArgs a, RefitLevels lv) {
+    for (uint32_t L = lv.count; L-- > 0;) {
+        for (uint32_t i = lv.start[L] + threadIdx.x; i < lv.start[L + 1]; i += kRefitThreads) refit_node(a, i);
+        __syncthreads();
+    }
 }
 
 // Flattened-BVH refit: record p takes its positions again from its BLAS record (v1.w
 // names the instance, v2.w the record in that instance's BLAS pool); the w words are
 // kept.  Raises the largest coordinate magnitude (one segment).
-__global__ void k_refit_flat_records(const InstanceRecord* inst, uint32_t n, float4* tri, uint32_t* seg_mag) {
-    uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    float4* t = tri + 3 * size_t(p);
-    const float4 t0 = t[0], t1 = t[1], t2 = t[2];
-    const uint32_t ii = __float_as_uint(t1.w) & ~kFlatOpaque, rec = __float_as_uint(t2.w);
-    const float4* src = inst[ii].tris + 3 * size_t(rec);
-    const float4 a = src[0], b = src[1], c = src[2];
-    t[0] = make_float4(a.x, a.y, a.z, t0.w);
-    t[1] = make_float4(b.x, b.y, b.z, t1.w);
-    t[2] = make_float4(c.x, c.y, c.z, t2.w);
-    const float3 m = fmax3(fmax3(mk3(fabsf(a.x), fabsf(a.y), fabsf(a.z)), mk3(fabsf(b.x), fabsf(b.y), fabsf(b.z))),
-                           mk3(fabsf(c.x), fabsf(c.y), fabsf(c.z)));
-    const float mag = fmaxf(m.x, fmaxf(m.y, m.z));
-    if (isfinite(mag)) atomicMax(seg_mag, __float_as_uint(mag));
+__global__ __launch_bounds__(kBlock) void k_refit_flat_records(const InstanceRecord* inst, uint32_t n, uint32_t span,
+                                                               float4* tri, uint32_t* seg_mag) {
+    const uint32_t base = blockIdx.x * span, end = base + min(span, n - base);
+    uint32_t most = 0;
+    for (uint32_t p = base + threadIdx.x; p < end; p += kBlock) {
+        float4* t = tri + 3 * size_t(p);
+        const float4 t0 = t[0], t1 = t[1], t2 = t[2];
+        const uint32_t ii = __float_as_uint(t1.w) & ~kFlatOpaque, rec = __float_as_uint(t2.w);
+        const float4* src = inst[ii].tris + 3 * size_t(rec);
+        const float4 a = src[0], b = src[1], c = src[2];
+        t[0] = make_float4(a.x, a.y, a.z, t0.w);
+        t[1] = make_float4(b.x, b.y, b.z, t1.w);
+        t[2] = make_float4(c.x, c.y, c.z, t2.w);
+        most = max(most, tri_mag(xyz(a), xyz(b), xyz(c)));
+    }
+    raise_block(seg_mag, most);
 }
 
 // Largest finite coordinate magnitude of a set of leaf boxes (one segment).
-__global__ void k_box_mag(const float4* lo, const float4* hi, uint32_t n, uint32_t* seg_mag) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float v[6] = {lo[i].x, lo[i].y, lo[i].z, hi[i].x, hi[i].y, hi[i].z};
+__global__ __launch_bounds__(kBlock) void k_box_mag(const float4* lo, const float4* hi, uint32_t n, uint32_t span,
+                                                    uint32_t* seg_mag) {
+    const uint32_t base = blockIdx.x * span, end = base + min(span, n - base);
     float m = 0.f;
-    for (int k = 0; k < 6; k++)
-        if (isfinite(v[k])) m = fmaxf(m, fabsf(v[k]));
-    atomicMax(seg_mag, __float_as_uint(m));
-}
-
-__global__ void k_iota(uint32_t* out, uint32_t n) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = i;
-}
-
-// Root bounds of every BLAS (padded), as the build reports them; 0 for an empty one.
-__global__ void k_refit_bounds(BlasDesc* descs, uint32_t nseg, const float* node_box, const uint32_t* seg_mag) {
-    uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nseg) return;
-    const float* b = node_box + 6 * size_t(s);
-    const float pad = __uint_as_float(seg_mag[s]) * 9.5367431640625e-07f + 1e-30f;
-    const bool empty = !(b[0] <= b[3]);
-    for (int k = 0; k < 3; k++) {
-        descs[s].bounds[k] = empty ? 0.f : b[k] - pad;
-        descs[s].bounds[3 + k] = empty ? 0.f : b[3 + k] + pad;
+    for (uint32_t i = base + threadIdx.x; i < end; i += kBlock) {
+        const float v[6] = {lo[i].x, lo[i].y, lo[i].z, hi[i].x, hi[i].y, hi[i].z};
+        for (int k = 0; k < 6; k++)
+            if (isfinite(v[k])) m = fmaxf(m, fabsf(v[k]));
     }
+    raise_block(seg_mag, __float_as_uint(m));
 }
 
 }  // namespace
@@ -1787,33 +1854,71 @@ int lbvh_build(hipStream_t st, const float4* d_lo, const float4* d_hi, uint32_t 
 }
 
 namespace {
-// RAII bundle of temporary device buffers (refits).
-struct Scratch {
-    std::vector<void*> ptrs;
-    ~Scratch() {
-        for (void* p : ptrs) (void)hipFree(p);
+bool levels_match(const std::vector<uint32_t>& level_start, uint32_t nseg, uint32_t num_nodes) {
+    return level_start.size() >= 2 && level_start.front() == 0u && level_start[1] == nseg && level_start.back() == num_nodes;
+}
+
+// Refits every level, the deepest first; a.node_seg and a.node_box come from s.
+int refit_levels(hipStream_t st, ScratchPool& s, RefitArgs a, uint32_t num_nodes, const std::vector<uint32_t>& level_start,
+                 std::string* err) {
+    a.node_seg = s.alloc<uint32_t>(num_nodes);
+    a.node_box = s.alloc<float>(6 * size_t(num_nodes));
+    if (!a.node_seg || !a.node_box) {
+        *err = "out of device memory";
+        return int(hipErrorOutOfMemory);
     }
-    template <class T> T* alloc(size_t count) {
-        void* p = nullptr;
-        if (hipMalloc(&p, count * sizeof(T) + 16) != hipSuccess) return nullptr;
-        ptrs.push_back(p);
-        return (T*)p;
+    for (size_t L = level_start.size() - 1; L > 0;) {
+        const uint32_t c = level_start[L];
+        size_t top = L;  // levels top..L-1 are small
+        while (top > 0 && L - top < size_t(kRefitLevels) && level_start[top] - level_start[top - 1] <= kRefitSmall) top--;
+        if (top < L) {
+            RefitLevels lv;
+            lv.count = uint32_t(L - top);
+            for (uint32_t k = 0; k <= lv.count; k++) lv.start[k] = level_start[top + k];
+            hipLaunchKernelGGL(k_refit_levels, dim3(1), dim3(kRefitThreads), 0, st, a, lv);
+            L = top;
+        } else {
+            const uint32_t b = level_start[--L];
+            hipLaunchKernelGGL(k_refit_level, dim3(blocks_for(c - b, kBlock)), dim3(kBlock), 0, st, a, b, c);
+        }
     }
-};
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) *err = "refit launch";
+    return int(e);
+}
+
+// Refit of a one-segment tree (root node 0); seg_mag[0] is raised beforehand on the same
+// stream.  Writes the padded root box to bounds.
+int refit_tree(hipStream_t st, ScratchPool& s, RefitArgs a, uint32_t num_nodes, const std::vector<uint32_t>& level_start,
+               float bounds[6], std::string* err) {
+    a.nseg = 1u;
+    a.descs = s.alloc<BlasDesc>(1);
+    if (!a.descs) {
+        *err = "out of device memory";
+        return int(hipErrorOutOfMemory);
+    }
+    const int rc = refit_levels(st, s, a, num_nodes, level_start, err);
+    if (rc) return rc;
+    hipError_t e = hipMemcpyAsync(bounds, a.descs->bounds, sizeof(float) * 6, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) *err = "refit launch";
+    return int(e);
+}
 }  // namespace
+
+size_t refit_scratch_bytes(uint32_t num_nodes, uint32_t nseg, uint32_t boxes) {
+    return size_t(num_nodes) * 28 + size_t(nseg) * 4 + size_t(boxes) * 32 + 8192;
+}
 
 int lbvh_refit(hipStream_t st, const TriSegment* d_segs, uint32_t nseg, uint32_t n, float4* d_tri, QNode* d_nodes,
                uint32_t num_nodes, const std::vector<uint32_t>& level_start, BlasDesc* d_descs, uint32_t* d_bad,
-               std::string* err) {
-    if (level_start.size() < 2 || level_start.front() != 0u || level_start[1] != nseg || level_start.back() != num_nodes) {
+               ScratchPool& s, std::string* err) {
+    if (!levels_match(level_start, nseg, num_nodes)) {
         *err = "the pool's level table does not match its nodes";
         return int(hipErrorInvalidValue);
     }
-    Scratch s;
     uint32_t* seg_mag = s.alloc<uint32_t>(nseg);
-    uint32_t* node_seg = s.alloc<uint32_t>(num_nodes);
-    float* node_box = s.alloc<float>(6 * size_t(num_nodes));
-    if (!seg_mag || !node_seg || !node_box) {
+    if (!seg_mag) {
         *err = "out of device memory";
         return int(hipErrorOutOfMemory);
     }
@@ -1822,72 +1927,25 @@ int lbvh_refit(hipStream_t st, const TriSegment* d_segs, uint32_t nseg, uint32_t
         *err = "memset";
         return int(e);
     }
-    if (n) hipLaunchKernelGGL(k_refit_records, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, d_segs, nseg, n, d_tri,
-                              seg_mag, d_bad);
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(nseg, kBlock)), dim3(kBlock), 0, st, node_seg, nseg);
-    const size_t levels = level_start.size() - 1;
-    for (size_t L = 0; L < levels; L++) {
-        const uint32_t b = level_start[L], c = level_start[L + 1];
-        if (c > b) hipLaunchKernelGGL(k_refit_seg, dim3(blocks_for(c - b, kBlock)), dim3(kBlock), 0, st, d_nodes, b, c, node_seg);
-    }
-    for (size_t L = levels; L-- > 0;) {
-        const uint32_t b = level_start[L], c = level_start[L + 1];
-        if (c > b)
-            hipLaunchKernelGGL(k_refit_level<false>, dim3(blocks_for(c - b, kBlock)), dim3(kBlock), 0, st, d_nodes, b, c,
-                               (const float4*)d_tri, (const float4*)nullptr, (const float4*)nullptr, node_seg, seg_mag,
-                               node_box);
-    }
-    hipLaunchKernelGGL(k_refit_bounds, dim3(blocks_for(nseg, kBlock)), dim3(kBlock), 0, st, d_descs, nseg, node_box, seg_mag);
-    e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(st);  // the scratch is freed on return
-    if (e != hipSuccess) *err = "refit launch";
-    return int(e);
+    if (n) hipLaunchKernelGGL(k_refit_records, dim3(blocks_for(n, bounds_span(n))), dim3(kBlock), 0, st, d_segs, nseg, n,
+                              bounds_span(n), d_tri, seg_mag, d_bad);
+    RefitArgs a = {};
+    a.nodes = d_nodes;
+    a.nseg = nseg;
+    a.segs = d_segs;
+    a.tri = d_tri;
+    a.seg_mag = seg_mag;
+    a.descs = d_descs;
+    return refit_levels(st, s, a, num_nodes, level_start, err);
 }
 
-namespace {
-// Bottom-up refit of a one-segment tree (root node 0) whose leaf entries index
-// triangle records (tri) or boxes (leaf_lo / leaf_hi); `prepare` has raised
-// seg_mag[0] beforehand on the same stream.  Writes the padded root box to bounds.
-int refit_tree(hipStream_t st, Scratch& s, QNode* d_nodes, uint32_t num_nodes, const std::vector<uint32_t>& level_start,
-               const float4* tri, const float4* leaf_lo, const float4* leaf_hi, uint32_t* seg_mag, float bounds[6],
-               std::string* err) {
-    if (level_start.size() < 2 || level_start.front() != 0u || level_start[1] != 1u || level_start.back() != num_nodes) {
+int lbvh_refit_flat(hipStream_t st, const InstanceRecord* d_inst, uint32_t n, float4* d_tri, QNode* d_nodes,
+                    uint32_t num_nodes, const std::vector<uint32_t>& level_start, float bounds[6], ScratchPool& s,
+                    std::string* err) {
+    if (!levels_match(level_start, 1u, num_nodes)) {
         *err = "the tree's level table does not match its nodes";
         return int(hipErrorInvalidValue);
     }
-    uint32_t* node_seg = s.alloc<uint32_t>(num_nodes);
-    float* node_box = s.alloc<float>(6 * size_t(num_nodes));
-    BlasDesc* desc = s.alloc<BlasDesc>(1);
-    if (!node_seg || !node_box || !desc) {
-        *err = "out of device memory";
-        return int(hipErrorOutOfMemory);
-    }
-    hipError_t e = hipMemsetAsync(node_seg, 0, sizeof(uint32_t) * num_nodes, st);
-    const size_t levels = level_start.size() - 1;
-    for (size_t L = levels; e == hipSuccess && L-- > 0;) {
-        const uint32_t b = level_start[L], c = level_start[L + 1];
-        if (c <= b) continue;
-        if (leaf_lo)
-            hipLaunchKernelGGL(k_refit_level<true>, dim3(blocks_for(c - b, kBlock)), dim3(kBlock), 0, st, d_nodes, b, c,
-                               (const float4*)nullptr, leaf_lo, leaf_hi, node_seg, seg_mag, node_box);
-        else
-            hipLaunchKernelGGL(k_refit_level<false>, dim3(blocks_for(c - b, kBlock)), dim3(kBlock), 0, st, d_nodes, b,
-                               c, tri, (const float4*)nullptr, (const float4*)nullptr, node_seg, seg_mag, node_box);
-    }
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_refit_bounds, dim3(1), dim3(kBlock), 0, st, desc, 1u, node_box, seg_mag);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipMemcpyAsync(bounds, desc->bounds, sizeof(float) * 6, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);  // the scratch is freed on return
-    if (e != hipSuccess) *err = "refit launch";
-    return int(e);
-}
-}  // namespace
-
-int lbvh_refit_flat(hipStream_t st, const InstanceRecord* d_inst, uint32_t n, float4* d_tri, QNode* d_nodes,
-                    uint32_t num_nodes, const std::vector<uint32_t>& level_start, float bounds[6], std::string* err) {
-    Scratch s;
     uint32_t* seg_mag = s.alloc<uint32_t>(1);
     if (!seg_mag) {
         *err = "out of device memory";
@@ -1898,14 +1956,21 @@ int lbvh_refit_flat(hipStream_t st, const InstanceRecord* d_inst, uint32_t n, fl
         *err = "memset";
         return int(e);
     }
-    if (n) hipLaunchKernelGGL(k_refit_flat_records, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, d_inst, n, d_tri,
-                              seg_mag);
-    return refit_tree(st, s, d_nodes, num_nodes, level_start, d_tri, nullptr, nullptr, seg_mag, bounds, err);
+    if (n) hipLaunchKernelGGL(k_refit_flat_records, dim3(blocks_for(n, bounds_span(n))), dim3(kBlock), 0, st, d_inst, n,
+                              bounds_span(n), d_tri, seg_mag);
+    RefitArgs a = {};
+    a.nodes = d_nodes;
+    a.tri = d_tri;
+    a.seg_mag = seg_mag;
+    return refit_tree(st, s, a, num_nodes, level_start, bounds, err);
 }
 
 int lbvh_refit_instances(hipStream_t st, const InstanceRecord* d_inst, uint32_t n, QNode* d_nodes, uint32_t num_nodes,
-                         const std::vector<uint32_t>& level_start, float bounds[6], std::string* err) {
-    Scratch s;
+                         const std::vector<uint32_t>& level_start, float bounds[6], ScratchPool& s, std::string* err) {
+    if (!levels_match(level_start, 1u, num_nodes)) {
+        *err = "the tree's level table does not match its nodes";
+        return int(hipErrorInvalidValue);
+    }
     uint32_t* seg_mag = s.alloc<uint32_t>(1);
     float4* lo = s.alloc<float4>(n + 1);
     float4* hi = s.alloc<float4>(n + 1);
@@ -1923,8 +1988,14 @@ int lbvh_refit_instances(hipStream_t st, const InstanceRecord* d_inst, uint32_t 
         *err = "instance boxes";
         return rc;
     }
-    if (n) hipLaunchKernelGGL(k_box_mag, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, lo, hi, n, seg_mag);
-    return refit_tree(st, s, d_nodes, num_nodes, level_start, nullptr, lo, hi, seg_mag, bounds, err);
+    if (n) hipLaunchKernelGGL(k_box_mag, dim3(blocks_for(n, bounds_span(n))), dim3(kBlock), 0, st, lo, hi, n, bounds_span(n),
+                              seg_mag);
+    RefitArgs a = {};
+    a.nodes = d_nodes;
+    a.leaf_lo = lo;
+    a.leaf_hi = hi;
+    a.seg_mag = seg_mag;
+    return refit_tree(st, s, a, num_nodes, level_start, bounds, err);
 }
 
 }  // namespace rt

@@ -4,6 +4,7 @@ segments that share tiles.  Every tree passes the validity walk (bit-exact: ever
 in exactly one leaf, inside every box on its path)."""
 import numpy as np
 import pytest
+import torch
 
 from rustracer_amd import bvhcheck, rt
 from rustracer_amd import layouts as L
@@ -81,3 +82,27 @@ def test_deep_paths_between_tiles(gpu_ctx, tiles):
     cam = S.cornell_sphere().ubo
     sc = b.finish("deep", S.make_instances([(None, g)]), [S.point_light((0, 3, 0), 1.0)], [L.default_dlight()], cam, 8, 8)
     _check(gpu_ctx, sc)
+
+
+@pytest.mark.parametrize("counts", [[3], [0, 5, 0], [1] * 700, [2, 1, 300, 1, 1, 255, 513, 1] * 3, [4096] * 5, [70001]])
+def test_refit_there_and_back(gpu_ctx, counts):
+    """Refit to other vertices and back gives the built nodes bit for bit: boxes, padding
+    by the segment's largest coordinate, quantising."""
+    sc = _scene(counts, 9, "cloud")
+    ds = G.DeviceScene(gpu_ctx, sc)
+
+    def nodes():
+        return [rt.read_nodes(gpu_ctx, i).tobytes() for i in (ds.blases[0].info(), ds.tlas.flat_info(), ds.tlas.info())
+                if i.num_nodes]
+
+    built = nodes()
+    moved = ds.buffers.vertices.clone()
+    v = moved.view(torch.float32).reshape(-1, L.VERTEX.itemsize // 4)
+    k = L.VERTEX.fields["pos"][1] // 4
+    v[:, k:k + 3] *= -3.0
+    rt.refit_as(gpu_ctx, sc, ds.buffers, ds.blases, vertices=moved, tlas=ds.tlas)
+    assert all(e == [] for e in bvhcheck.check_blases(gpu_ctx, ds.blases, counts))
+    assert not bvhcheck.check_tlas(gpu_ctx, ds.tlas, len(counts))
+    assert nodes()[0] != built[0]
+    rt.refit_as(gpu_ctx, sc, ds.buffers, ds.blases, tlas=ds.tlas)
+    assert nodes() == built
