@@ -689,11 +689,16 @@ __device__ inline D3 render_pixel(const FrameArgs& fa, uint32_t x, uint32_t y, u
 // A lane of a persistent kernel that runs pixels' raygen loops (run_samples: the
 // same operations on the same values, in the same order) with its traversals
 // stepped rather than run to completion.  The kernel's waves alternate: step the
-// lanes that trace (path or shadow ray) while at least half of the lanes that hold
-// a pixel do, then the others advance together (shading, next ray, next sample), so
-// no lane waits each bounce for the slowest traversal of its wave.
+// lanes that trace (path or shadow ray) while at least trace_keep of the lanes that
+// hold a pixel do, then the others advance together (shading, next ray, next sample),
+// so no lane waits each bounce for the slowest traversal of its wave.
 enum : uint32_t { kLaneIdle = 0, kLaneExt, kLaneShadow, kLaneShade, kLaneNext, kLaneDone };
 enum : uint32_t { kAfterExt = 0, kAfterDone, kAfterNext };  // what follows a shadow ray
+
+// 3/16 of them: an advance costs the wave several traversal steps whatever its lanes, so
+// it waits for company (957x539, 4 samples: 12/16 5.6 ms, 8/16 4.75, 4/16 4.49, 3/16
+// 4.50, 1/16 4.85; 128x128: 0.55, 0.47, 0.42, 0.40, 0.39).
+__device__ inline uint32_t trace_keep(uint64_t holding) { return (uint32_t(__popcll(holding)) * 3u + 15u) / 16u; }
 
 // The ray of a lane's traversal: the path's fp64 ray, or the fp32 shadow ray.
 struct LaneRay {

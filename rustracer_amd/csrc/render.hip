@@ -61,11 +61,13 @@ __device__ inline void mega_pixel(const FrameArgs& fa, uint32_t x, uint32_t y, u
 // Persistent form: lanes take pixels from one counter (tile by tile, tiles in image
 // order) and run them as PathLanes, traversals stepped and the wave's shading done
 // together, so no lane waits each bounce for the slowest traversal of its wave; a
-// lane that finishes its pixel takes the next (one atomic per wave).
+// lane that finishes its pixel takes the next (one atomic per wave).  `lanes` lanes of each
+// wave take pixels (spread_lanes).
 template <bool kAnyHit, bool kStats>
-__global__ __launch_bounds__(kMegaBlock) void k_megakernel_persistent(FrameArgs fa, uint32_t* next_pixel) {
+__global__ __launch_bounds__(kMegaBlock) void k_megakernel_persistent(FrameArgs fa, uint32_t* next_pixel, uint32_t lanes) {
     __shared__ uint32_t s_stack[kStackDepth * kMegaBlock];
     uint32_t* const stack = s_stack + threadIdx.x;
+    const bool takes = __lane_id() < lanes;
     const uint32_t tiles_x = (fa.width + 7) / 8;
     const uint32_t items = tiles_x * ((fa.height + 7) / 8) * 64u;
     const bool heat = fa.o.out && fa.o.mapping == RT_MAPPING_HEAT;
@@ -75,7 +77,7 @@ __global__ __launch_bounds__(kMegaBlock) void k_megakernel_persistent(FrameArgs 
     bool exhausted = false;
     for (;;) {
         if (!exhausted) {
-            const uint32_t it = wave_fetch(ln.state == kLaneIdle, next_pixel, items, exhausted);
+            const uint32_t it = wave_fetch(takes && ln.state == kLaneIdle, next_pixel, items, exhausted);
             if (it != kEmpty) {
                 const uint32_t tile = it >> 6, within = it & 63u;
                 const uint32_t x = (tile % tiles_x) * 8 + (within & 7u);
@@ -88,7 +90,7 @@ __global__ __launch_bounds__(kMegaBlock) void k_megakernel_persistent(FrameArgs 
         }
         const uint64_t holding = __ballot(ln.state != kLaneIdle);
         if (!holding && exhausted) break;
-        const uint32_t keep = (uint32_t(__popcll(holding)) + 1u) / 2u;
+        const uint32_t keep = trace_keep(holding);
         while (keep && uint32_t(__popcll(__ballot(ln.tracing()))) >= keep) {
             if (ln.tracing()) {
                 AlphaAnyHit ah{&fa.sv, &fa.tlas, &ln.rng};
@@ -123,10 +125,11 @@ __global__ __launch_bounds__(kMegaBlock) void k_megakernel(FrameArgs fa) {
 
 template <bool kAnyHit>
 __global__ __launch_bounds__(kMegaBlock) void k_ray_queries(TlasView tl, SceneView sv, const rt_ray* rays, uint32_t n,
-                                                             uint32_t flags, rt_hit* hits, uint32_t seed_b) {
+                                                             uint32_t flags, rt_hit* hits, uint32_t seed_b,
+                                                             uint32_t lanes) {
     __shared__ uint32_t s_stack[kStackDepth * kMegaBlock];
-    uint32_t i = blockIdx.x * kMegaBlock + threadIdx.x;
-    if (i >= n) return;
+    uint32_t i = (blockIdx.x * (kMegaBlock / 64) + (threadIdx.x >> 6)) * lanes + __lane_id();
+    if (__lane_id() >= lanes || i >= n) return;
     rt_ray r = rays[i];
     Rng4 rng{i, 0u, seed_b, 0u};
     AlphaAnyHit ah{&sv, &tl, &rng};
@@ -154,10 +157,10 @@ __global__ __launch_bounds__(kMegaBlock) void k_ray_queries(TlasView tl, SceneVi
 }
 
 template <bool kAnyHit>
-__global__ __launch_bounds__(kMegaBlock) void k_primary(FrameArgs fa, rt_hit* hits) {
+__global__ __launch_bounds__(kMegaBlock) void k_primary(FrameArgs fa, rt_hit* hits, uint32_t lanes) {
     __shared__ uint32_t s_stack[kStackDepth * kMegaBlock];
-    uint32_t i = blockIdx.x * kMegaBlock + threadIdx.x;
-    if (i >= fa.width * fa.height) return;
+    uint32_t i = (blockIdx.x * (kMegaBlock / 64) + (threadIdx.x >> 6)) * lanes + __lane_id();
+    if (__lane_id() >= lanes || i >= fa.width * fa.height) return;
     uint32_t x = i % fa.width, y = i / fa.width;
     Rng4 rng_a{x, y, fa.frame_count, 0u};
     Rng4 rng_b{x, y, fa.seed_b, 0u};
@@ -209,6 +212,20 @@ static uint32_t resident_grid(const void* f) {
     return g;
 }
 
+// SIMDs of the current device: four to a CU.
+static uint32_t simds() {
+    int dev = 0, cus = 0;
+    (void)hipGetDevice(&dev);
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
+    return uint32_t(cus) * 4u;
+}
+
+// Workgroups whose waves take `lanes` items each.
+static uint64_t blocks_of(uint64_t n, uint32_t lanes) {
+    const uint64_t per = uint64_t(lanes) * (kMegaBlock / 64);
+    return (n + per - 1) / per;
+}
+
 int launch_megakernel(const FrameArgs& fa, hipStream_t st, bool any_hit, bool stats, StageTimer* tm,
                       uint32_t* next_pixel) {
     uint32_t tiles = ((fa.width + 15) / 16) * ((fa.height + 7) / 8);
@@ -224,14 +241,16 @@ int launch_megakernel(const FrameArgs& fa, hipStream_t st, bool any_hit, bool st
                                          : (const void*)k_megakernel_persistent<true, false>)
                                 : (stats ? (const void*)k_megakernel_persistent<false, true>
                                          : (const void*)k_megakernel_persistent<false, false>);
-        // no more workgroups than there are pixel tiles to start on
-        const uint32_t g = std::min(resident_grid(f), tiles);
+        // no more workgroups than there are pixels to start on
+        const uint32_t items = ((fa.width + 7) / 8) * ((fa.height + 7) / 8) * 64u;
+        const uint32_t lanes = spread_lanes(items, simds());
+        const uint32_t g = std::min(resident_grid(f), uint32_t(blocks_of(items, lanes)));
         if (any_hit) {
-            if (stats) hipLaunchKernelGGL((k_megakernel_persistent<true, true>), dim3(g), dim3(kMegaBlock), 0, st, fa, next_pixel);
-            else hipLaunchKernelGGL((k_megakernel_persistent<true, false>), dim3(g), dim3(kMegaBlock), 0, st, fa, next_pixel);
+            if (stats) hipLaunchKernelGGL((k_megakernel_persistent<true, true>), dim3(g), dim3(kMegaBlock), 0, st, fa, next_pixel, lanes);
+            else hipLaunchKernelGGL((k_megakernel_persistent<true, false>), dim3(g), dim3(kMegaBlock), 0, st, fa, next_pixel, lanes);
         } else {
-            if (stats) hipLaunchKernelGGL((k_megakernel_persistent<false, true>), dim3(g), dim3(kMegaBlock), 0, st, fa, next_pixel);
-            else hipLaunchKernelGGL((k_megakernel_persistent<false, false>), dim3(g), dim3(kMegaBlock), 0, st, fa, next_pixel);
+            if (stats) hipLaunchKernelGGL((k_megakernel_persistent<false, true>), dim3(g), dim3(kMegaBlock), 0, st, fa, next_pixel, lanes);
+            else hipLaunchKernelGGL((k_megakernel_persistent<false, false>), dim3(g), dim3(kMegaBlock), 0, st, fa, next_pixel, lanes);
         }
     } else if (any_hit) {
         if (stats) hipLaunchKernelGGL((k_megakernel<true, true>), dim3(tiles), dim3(kMegaBlock), 0, st, fa);
@@ -251,18 +270,20 @@ int launch_megakernel(const FrameArgs& fa, hipStream_t st, bool any_hit, bool st
 int launch_ray_queries(const TlasView& tl, const SceneView& sv, const rt_ray* rays, uint32_t n, uint32_t flags,
                        rt_hit* hits, uint32_t seed_b, hipStream_t st, bool any_hit) {
     if (n == 0) return 0;
-    uint32_t nb = (n + kMegaBlock - 1) / kMegaBlock;
-    if (any_hit) hipLaunchKernelGGL((k_ray_queries<true>), dim3(nb), dim3(kMegaBlock), 0, st, tl, sv, rays, n, flags, hits, seed_b);
-    else hipLaunchKernelGGL((k_ray_queries<false>), dim3(nb), dim3(kMegaBlock), 0, st, tl, sv, rays, n, flags, hits, seed_b);
+    const uint32_t lanes = spread_lanes(n, simds());
+    const dim3 grid{uint32_t(blocks_of(n, lanes))};
+    if (any_hit) hipLaunchKernelGGL((k_ray_queries<true>), grid, dim3(kMegaBlock), 0, st, tl, sv, rays, n, flags, hits, seed_b, lanes);
+    else hipLaunchKernelGGL((k_ray_queries<false>), grid, dim3(kMegaBlock), 0, st, tl, sv, rays, n, flags, hits, seed_b, lanes);
     return int(hipGetLastError());
 }
 
 int launch_primary(const FrameArgs& fa, rt_hit* hits, hipStream_t st, bool any_hit) {
     uint32_t n = fa.width * fa.height;
     if (n == 0) return 0;
-    uint32_t nb = (n + kMegaBlock - 1) / kMegaBlock;
-    if (any_hit) hipLaunchKernelGGL((k_primary<true>), dim3(nb), dim3(kMegaBlock), 0, st, fa, hits);
-    else hipLaunchKernelGGL((k_primary<false>), dim3(nb), dim3(kMegaBlock), 0, st, fa, hits);
+    const uint32_t lanes = spread_lanes(n, simds());
+    const dim3 grid{uint32_t(blocks_of(n, lanes))};
+    if (any_hit) hipLaunchKernelGGL((k_primary<true>), grid, dim3(kMegaBlock), 0, st, fa, hits, lanes);
+    else hipLaunchKernelGGL((k_primary<false>), grid, dim3(kMegaBlock), 0, st, fa, hits, lanes);
     return int(hipGetLastError());
 }
 

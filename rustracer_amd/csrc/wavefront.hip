@@ -403,14 +403,16 @@ __global__ __launch_bounds__(kWfBlock) void k_wf_shade(Frames fr, WfArrays a, co
 // samples (the megakernel's loop from the slot's state), then writes the pixel.  Its
 // lanes are PathLanes: traversals stepped, the wave's shading done together, and a
 // lane that finishes its pixel takes the next queue entry (one atomic per wave, the
-// trace cursor, which the last shade cleared).
+// trace cursor, which the last shade cleared).  `lanes` lanes of each wave take entries
+// (spread_lanes).
 constexpr int kFinishBlock = 128;
 
 template <class Frames, bool kAnyHit, bool kStats>
 __global__ __launch_bounds__(kFinishBlock) void k_wf_finish(Frames fr, WfArrays a, const uint32_t* q,
                                                             const uint32_t* n_e_in, const uint32_t* qs,
-                                                            const uint32_t* n_s_in) {
+                                                            const uint32_t* n_s_in, uint32_t lanes) {
     __shared__ uint32_t s_stack[kStackDepth * kFinishBlock];
+    const bool takes = __lane_id() < lanes;
     uint32_t* const stack = s_stack + threadIdx.x;
     const uint32_t n_e = *n_e_in, n = n_e + *n_s_in;
     PathCounters pc;
@@ -420,7 +422,7 @@ __global__ __launch_bounds__(kFinishBlock) void k_wf_finish(Frames fr, WfArrays 
     for (;;) {
         // lanes without a pixel take the next entry of q, then of qs (its retiring ones)
         if (!exhausted) {
-            const uint32_t i = wave_fetch(ln.state == kLaneIdle, a.counts + kCursor, n, exhausted);
+            const uint32_t i = wave_fetch(takes && ln.state == kLaneIdle, a.counts + kCursor, n, exhausted);
             if (i != kEmpty) {
                 const uint32_t entry = i < n_e ? q[i] : qs[i - n_e];
                 if (i < n_e || (entry & kRetireBit)) {  // a shadow entry without the bit has a path entry too
@@ -447,7 +449,7 @@ __global__ __launch_bounds__(kFinishBlock) void k_wf_finish(Frames fr, WfArrays 
         }
         const uint64_t holding = __ballot(ln.state != kLaneIdle);
         if (!holding && exhausted) break;
-        const uint32_t keep = (uint32_t(__popcll(holding)) + 1u) / 2u;
+        const uint32_t keep = trace_keep(holding);
         while (keep && uint32_t(__popcll(__ballot(ln.tracing()))) >= keep) {
             if (ln.tracing()) {
                 const FrameArgs& fa = fr.frame(f);
@@ -532,7 +534,8 @@ __global__ void k_zero_counts(uint32_t* c) {
 template <class Frames> struct Kernels {
     using TraceFn = void (*)(Frames, WfArrays, const uint32_t*, const uint32_t*, const uint32_t*, const uint32_t*,
                              uint32_t*, uint32_t*);
-    using FinishFn = void (*)(Frames, WfArrays, const uint32_t*, const uint32_t*, const uint32_t*, const uint32_t*);
+    using FinishFn = void (*)(Frames, WfArrays, const uint32_t*, const uint32_t*, const uint32_t*, const uint32_t*,
+                              uint32_t);
     static FinishFn finish(bool ah, bool st) {
         return ah ? (st ? k_wf_finish<Frames, true, true> : k_wf_finish<Frames, true, false>)
                   : (st ? k_wf_finish<Frames, false, true> : k_wf_finish<Frames, false, false>);
@@ -831,9 +834,11 @@ int run_wavefront(WavefrontState* ws, const std::vector<SlotSet<Frames>>& sets, 
             } else if (live < ws->finish_below && !tm) {
                 // the paths left after chunk c (at most `live`) end in one launch
                 const typename K::FinishFn k_finish = K::finish(any_hit, stats);
-                const uint32_t blocks = std::min((live + kFinishBlock - 1) / kFinishBlock, 65535u);
+                const uint32_t lanes = spread_lanes(uint64_t(live) * nsets, uint32_t(ws->cus) * 4u);
+                const uint32_t per = lanes * (kFinishBlock / 64);
+                const uint32_t blocks = std::min((live + per - 1) / per, 65535u);
                 hipLaunchKernelGGL(k_finish, dim3(blocks), dim3(kFinishBlock), 0, stream_of(g), sets[g].fr, sets[g].a,
-                                   sets[g].a.q0, sets[g].a.counts, sets[g].a.qs1, shadow_count(sets[g].a, 1));
+                                   sets[g].a.q0, sets[g].a.counts, sets[g].a.qs1, shadow_count(sets[g].a, 1), lanes);
                 e = hipGetLastError();
                 if (e != hipSuccess) {
                     *err = "launch k_wf_finish";
