@@ -578,11 +578,11 @@ struct WavefrontState {
     int cus = 0;
     std::unordered_map<const void*, uint32_t> grids;  // persistent grid per kernel (occupancy x CUs)
     // grid of a persistent launch of kernel `f`: as many blocks as can be resident
-    uint32_t grid_for(const void* f) {
+    uint32_t grid_for(const void* f, int block = kWfBlock) {
         auto it = grids.find(f);
         if (it != grids.end()) return it->second;
         int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, kWfBlock, 0) != hipSuccess || per_cu < 1) per_cu = 4;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, block, 0) != hipSuccess || per_cu < 1) per_cu = 4;
         uint32_t g = uint32_t(std::max(cus, 1)) * uint32_t(per_cu);
         grids.emplace(f, g);
         return g;
@@ -728,6 +728,19 @@ int run_wavefront(WavefrontState* ws, const std::vector<SlotSet<Frames>>& sets, 
             if (marks) mark(stage);
         });
     };
+    const typename K::FinishFn k_finish = K::finish(any_hit, stats);
+    // A set that starts with few paths ends in the finishing launch at once, without the two
+    // chunks of iterations that pass before its count is known (256x256 pixels, 4 samples:
+    // 2.96 ms with them, 1.87 without; 72x72, 1 sample 1.65 and 0.40).  The line is at two
+    // rounds of the chip's lanes for all the sets' paths (360x360 pixels of an opaque scene,
+    // 32 samples, 1.98 rounds: 34 ms in iterations, 24 in one launch), and at one round
+    // where hits are tested for alpha: rays through many instances vary most (360x360: 88 ms
+    // in iterations, 102 in one launch; 256x256: 28.5 and 25.5).
+    const uint64_t round = uint64_t(ws->grid_for((const void*)k_finish, kFinishBlock)) * kFinishBlock;
+    const uint64_t direct = any_hit ? round : 2 * round;
+    bool alive[kMaxStreams], any_alive = false;
+    for (int g = 0; g < kMaxStreams; g++)
+        alive[g] = g < nsets && (tm || sets[g].nslots >= ws->finish_below || uint64_t(sets[g].nslots) * nsets > direct);
     static_assert(kCheckEvery % 2 == 0, "a chunk ends on queue 0");
     const bool graph = ws->use_graph && !tm;
     if (graph) {
@@ -741,6 +754,7 @@ int run_wavefront(WavefrontState* ws, const std::vector<SlotSet<Frames>>& sets, 
             }
         }
         for (int g = 0; g < nsets; g++) {
+            if (!alive[g]) continue;
             e = hipStreamBeginCapture(ws->cap_stream, hipStreamCaptureModeThreadLocal);
             if (e != hipSuccess) {
                 *err = "hipStreamBeginCapture";
@@ -790,10 +804,25 @@ int run_wavefront(WavefrontState* ws, const std::vector<SlotSet<Frames>>& sets, 
         *err = "launch k_wf_init";
         rc = int(e);
     }
+    auto finish = [&](int g, uint32_t live) {
+        const uint32_t lanes = spread_lanes(uint64_t(live) * nsets, uint32_t(ws->cus) * 4u);
+        const uint32_t per = lanes * (kFinishBlock / 64);
+        const uint32_t blocks = std::min((live + per - 1) / per, 65535u);
+        hipLaunchKernelGGL(k_finish, dim3(blocks), dim3(kFinishBlock), 0, stream_of(g), sets[g].fr, sets[g].a,
+                           sets[g].a.q0, sets[g].a.counts, sets[g].a.qs1, shadow_count(sets[g].a, 1), lanes);
+    };
     const uint64_t max_chunks = max_steps / kCheckEvery + 2;
-    bool alive[kMaxStreams];
-    for (int g = 0; g < kMaxStreams; g++) alive[g] = g < nsets;
-    for (uint64_t c = 0; rc == 0; c++) {
+    for (int g = 0; g < nsets && rc == 0; g++) {
+        any_alive = any_alive || alive[g];
+        if (alive[g]) continue;
+        finish(g, sets[g].nslots);
+        e = hipGetLastError();
+        if (e != hipSuccess) {
+            *err = "launch k_wf_finish";
+            rc = int(e);
+        }
+    }
+    for (uint64_t c = 0; rc == 0 && any_alive; c++) {
         // enqueue chunk c of every live set, then its live-path count read-back
         for (int g = 0; g < nsets && rc == 0; g++) {
             if (!alive[g]) continue;
@@ -833,12 +862,7 @@ int run_wavefront(WavefrontState* ws, const std::vector<SlotSet<Frames>>& sets, 
                 alive[g] = false;
             } else if (live < ws->finish_below && !tm) {
                 // the paths left after chunk c (at most `live`) end in one launch
-                const typename K::FinishFn k_finish = K::finish(any_hit, stats);
-                const uint32_t lanes = spread_lanes(uint64_t(live) * nsets, uint32_t(ws->cus) * 4u);
-                const uint32_t per = lanes * (kFinishBlock / 64);
-                const uint32_t blocks = std::min((live + per - 1) / per, 65535u);
-                hipLaunchKernelGGL(k_finish, dim3(blocks), dim3(kFinishBlock), 0, stream_of(g), sets[g].fr, sets[g].a,
-                                   sets[g].a.q0, sets[g].a.counts, sets[g].a.qs1, shadow_count(sets[g].a, 1), lanes);
+                finish(g, live);
                 e = hipGetLastError();
                 if (e != hipSuccess) {
                     *err = "launch k_wf_finish";
