@@ -560,7 +560,8 @@ void rt_destroy_blas(rt_ctx* ctx, rt_blas blas) {
     auto it = ctx->blas.find(blas);
     if (it == ctx->blas.end()) return;
     DeviceGuard g(ctx->device);
-    (void)hipStreamSynchronize(ctx->stream);
+    // work in flight may read the batch's memory: wait before the last holder lets go of it
+    if (it->second.pool.use_count() == 1) (void)hipStreamSynchronize(ctx->stream);
     ctx->blas_by_addr.erase(uint64_t(uintptr_t(it->second.d_desc)));
     ctx->blas.erase(it);
 }

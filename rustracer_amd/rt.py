@@ -335,20 +335,39 @@ class Blas:
             pass
 
 
+def _max_vertices(geo, indices):
+    """Largest index of each geometry's run of the index buffer, 0 for an empty one."""
+    first = geo["index_offset"].astype(np.int64)
+    count = 3 * geo["prim_count"].astype(np.int64)
+    out = np.zeros(len(geo), np.uint32)
+    some = np.nonzero(count)[0]
+    start, end = first[some], (first + count)[some]
+    if len(some) and np.array_equal(start[1:], end[:-1]) and end[-1] <= len(indices):
+        out[some] = np.maximum.reduceat(indices[:end[-1]], start)  # runs that follow one another
+    else:
+        for k, a, b in zip(some, start, end):
+            out[k] = indices[a:b].max()
+    return out
+
+
 def blas_inputs(scene, buffers, vertices=None):
     """primitive_to_vk_geometry (acceleration_structures.rs:17-76) for every geometry id;
     `vertices` (a device tensor in the vertex layout) replaces the vertex buffer, as the
     reference uses its animation buffer for skinned geometry (:23-27)."""
     geo = scene.geometries
     ins = (BlasInput * len(geo))()
-    vb = (buffers.vertices if vertices is None else vertices).data_ptr()
-    ib = buffers.indices.data_ptr()
-    for g in range(len(geo)):
-        first_vertex, index_offset, count, opaque = (int(x) for x in geo[g])
-        idx = scene.indices[index_offset:index_offset + 3 * count]
-        max_vertex = int(idx.max()) if count else 0
-        ins[g] = BlasInput(vb, L.VERTEX.itemsize, max_vertex, ib, first_vertex, 4 * index_offset, count,
-                           GEOMETRY_OPAQUE if opaque else 0)
+    if not len(geo):
+        return ins
+    # the records are filled as arrays: 1,951 geometries took 7 ms one by one, 0.6 so
+    rec = np.frombuffer(ins, np.dtype(BlasInput))
+    rec["vertex_data"] = (buffers.vertices if vertices is None else vertices).data_ptr()
+    rec["vertex_stride"] = L.VERTEX.itemsize
+    rec["max_vertex"] = _max_vertices(geo, scene.indices)
+    rec["index_data"] = buffers.indices.data_ptr()
+    rec["first_vertex"] = geo["first_vertex"]
+    rec["primitive_offset"] = 4 * geo["index_offset"]
+    rec["primitive_count"] = geo["prim_count"]
+    rec["geometry_flags"] = np.where(geo["opaque"], GEOMETRY_OPAQUE, 0)
     return ins
 
 
@@ -390,11 +409,21 @@ def skin_vertices(ctx, vertices_in, vertices_out, skins):
                                        n, C.c_void_p(skins.data_ptr()) if ns else None, ns))
 
 
+def _addresses(ctx, blases):
+    a = C.c_uint64()
+    ref, call = C.byref(a), ctx.lib.rt_blas_device_address
+    out = []
+    for b in blases:
+        b.ctx.check(call(b.ctx.handle, b.handle, ref))
+        out.append(a.value)
+    return out
+
+
 def create_top_as(ctx, scene, blases):
     """create_top_as (acceleration_structures.rs:136-249): the scene's instance records
     with the BLAS reference replaced by the BLAS device address, uploaded and built."""
     inst = np.array(scene.instances, copy=True)
-    addr = np.array([b.address() for b in blases], np.uint64)
+    addr = np.array(_addresses(ctx, blases), np.uint64)
     inst["acceleration_structure_reference"] = addr[scene.instances["acceleration_structure_reference"].astype(np.int64)]
     d_inst = to_device(inst)
     out = C.c_uint64()
