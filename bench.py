@@ -225,7 +225,7 @@ def adjoint_iteration(ctx, steps, warmup):
             "workload": "Cornell box 512x512, 16 spp, depth 4, 512^2 RGBA32F base-colour + metallic-roughness "
                         "parameter textures and the point light's intensity; forward in the faster mode (autotuned "
                         "wavefront or persistent megakernel, same image) + L2 gradient + path-replay adjoint (each "
-                        "sample traced again, per-wave LDS sums before the float atomics)"}
+                        "sample replayed from its hits, per-wave LDS sums before the float atomics)"}
 
 
 def dynamic_step(ctx, sc, buf, blases, steps):

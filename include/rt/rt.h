@@ -334,7 +334,7 @@ enum {
      * before the collapse to 4-wide nodes: bottom up, each node's treelet of up to
      * five subtrees is rebuilt as the binary tree of least surface-area-heuristic
      * cost over them (Karras & Aila, HPG 2013).  0: the Morton-order tree as
-     * emitted, built in less than half the time (for scenes rebuilt every frame).
+     * emitted, built in 0.6 of the time (for scenes rebuilt every frame).
      * Same hits.  Default 2. */
     RT_OPTION_BVH_TREELET_PASSES = 14
 };

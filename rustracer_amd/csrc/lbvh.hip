@@ -1,14 +1,15 @@
 // lbvh.hip — batched LBVH build for gfx950 (see lbvh.h).
 //
 // Pipeline per build (all on one stream):
-//   1. primitive boxes + per-segment centroid bounds (wave-reduced atomics)
+//   1. primitive boxes + per-segment bounds (reduced per workgroup before the atomics)
 //   2. 64-bit keys: segment id above an interleaved Morton code
 //   3. LSD radix sort, 8 bits per pass: LDS histogram, three-kernel scan, and an
-//      LDS-staged stable scatter that ranks keys with wave ballots
+//      LDS-staged stable scatter that ranks keys with wave ballots; small builds sort
+//      by rank in one launch
 //   4. Karras (HPG 2012) radix-tree emission, one thread per internal node
-//   5. bottom-up box fit with acquire/release counters
-//   6. top-down collapse into 4-wide nodes, one kernel launch per level.  With the
-//      SAH collapse (default), the box-fit pass also solves, bottom-up, for every
+//   5. bottom-up passes over tiles of the tree in LDS: treelet restructuring, boxes
+//   6. top-down collapse into 4-wide quantised nodes, two launches per level.  With the
+//      SAH collapse (default), the bottom-up pass also solves, bottom-up, for every
 //      binary node n and every number of slots i = 1..4 it may take in its parent's
 //      wide node, the least surface-area-heuristic cost of its subtree
 //        C(n, 1) = min(leaf: c_tri |n| A(n) if |n| <= leaf size,
