@@ -246,19 +246,21 @@ int rt_trace_rays_batch(rt_ctx* ctx, const rt_batch_item* items, uint32_t count,
  *   - the intensity of directional light i, into d_grad_directional_intensity[i]
  *     (b->num_dlights floats, or NULL), through the miss shader's
  *     -cos * colour * intensity (RayTracing.rmiss:18-26).
- * Each sample is traced twice (path replay): once for its radiance and shadow
- * results, once more to differentiate it vertex by vertex; nothing else of the
- * path is stored.  Lobe choices, directions, sampling densities (the RIS light
+ * Each sample runs twice (path replay): once for its radiance and shadow results,
+ * once more to differentiate it vertex by vertex; of the path itself only the hits
+ * of its first bounces are kept, the others are traced again.  The gradient of an
+ * intensity is summed in fp64 over the frame and rounded once.  Lobe choices, directions, sampling densities (the RIS light
  * weight included) and Russian roulette are held at their forward values, so the
  * result is the derivative of the image's estimate with the sampling detached, for
  * the same bindings and UBO as the forward trace.  d_grad_accum is the device
  * array dLoss/d(accum), width * height * 4 floats (alpha ignored); pixels whose
  * gradient is zero are skipped.  At most 64 bounces, and ubo.debug == 1 (the legacy
  * materials) is not differentiated (RT_ERR_UNSUPPORTED for both).  With `stats`,
- * its ray and traversal counters count both passes, and grad_taps / grad_atomics
- * count the gradient contributions and the float atomics they became.  There is no
- * adjoint in the reference; it serves an optimisation loop around the trace that
- * record_raytracing_commands issues (crates/examples/gltf_viewer/src/main.rs:244-270). */
+ * both passes are traced in full and its ray and traversal counters count both, and
+ * grad_taps / grad_atomics count the gradient contributions and the atomics they
+ * became.  There is no adjoint in the reference; it serves an optimisation loop around
+ * the trace that record_raytracing_commands issues
+ * (crates/examples/gltf_viewer/src/main.rs:244-270). */
 int rt_trace_rays_adjoint(rt_ctx* ctx, rt_tlas tlas, const rt_bindings* b, const float* d_grad_accum,
                           uint32_t width, uint32_t height, float* const* grad_textures, float* d_grad_point_intensity,
                           float* d_grad_directional_intensity, rt_trace_stats* stats);

@@ -9,13 +9,15 @@ namespace rt {
 // results in a 64-bit mask.
 constexpr uint32_t kMaxAdjointBounces = 64;
 
-// Where the adjoint writes (all device memory; each entry may be NULL).
+// Where the adjoint writes (all device memory; each entry may be NULL, light_sums only
+// when both light gradients are).
 struct AdjointOut {
     float* const* grads;      // device array of num_textures pointers: gradient buffer of
                               // RGBA32F texture i (its texel layout), or NULL
     uint32_t num_textures;
     float* grad_plight;       // d/d intensity of point light i (num_plights floats)
     float* grad_dlight;       // d/d intensity of directional light i (num_dlights floats)
+    double* light_sums;       // scratch: num_plights + num_dlights sums (cleared on the stream here)
 };
 
 // Accumulates into `out` the gradient of sum(grad_accum * accum) over the frame `fa`

@@ -4,12 +4,14 @@
 // metallic-roughness materials, and to the intensities of the point and
 // directional lights.
 //
-// Path replay backpropagation (Vicini, Speierer & Jakob, SIGGRAPH 2021): nothing of
-// a path is stored between its two passes but its radiance and one bit per bounce.
+// Path replay backpropagation (Vicini, Speierer & Jakob, SIGGRAPH 2021): of a path, its
+// radiance, one bit per bounce and the hits of its first bounces (kKeptHits) are kept
+// between its two passes, whatever its length.
 // One lane per pixel at a time (persistent lanes taking pixels in turn); per sample:
 //   pass 1  the forward path (traversal, shading, shadow rays) gives the sample's
 //           radiance L and the shadow results (one bit per bounce);
-//   pass 2  the same path traced and shaded again from the same RNG state.  At
+//   pass 2  the same path shaded again from the same RNG state (and traced again beyond
+//           the kept hits).  At
 //           vertex k with throughput T_k, radiance added E_k and throughput factor
 //           M_k (T_{k+1} = T_k M_k), the radiance still to come is
 //             L_k = L - sum_{j<=k} T_j E_j = T_{k+1} R_{k+1},
@@ -25,13 +27,17 @@
 // Russian roulette are held at their forward values (detached sampling), so the
 // replay sees the forward paths exactly.
 //
-// Scatter.  A vertex's contributions (texel x channel, or light) are summed per
-// wave in an LDS table keyed by the target address before any float atomic: the
-// camera-ray vertices of a wave's 8x8 pixels and 16 samples share a few hundred
-// texels, and every lane's NEE adds to the same few lights.  The table is drained
-// into the gradient buffers with one atomic per key when it is half full at the end
-// of a sample, and at the end of the kernel; a key that finds no free slot within
-// a few probes goes to the atomics directly.
+// Scatter.  A vertex's texel contributions (texel x channel) are summed per wave in an
+// LDS table keyed by the target address before any float atomic: the camera-ray
+// vertices of a wave's 8x8 pixels and 16 samples share a few hundred texels.  The table
+// is drained into the gradient buffers with one atomic per key when it is half full at
+// the end of a sample, and at the end of the kernel; a key that finds no free slot
+// within a few probes goes to the atomics directly.
+//
+// Lights.  Every NEE vertex of the frame adds to the same few intensities, with either
+// sign, so their sums are kept in fp64 (per wave in LDS, then over the grid) and rounded
+// once: in fp32 the order of millions of additions moved the gradient of 512x512 pixels
+// by 1e-5 to 1e-3 of its value from one call to the next.
 //
 // Follows the raygen loop of crates/examples/gltf_viewer/shaders/RayTracing.rgen
 // (:85-128), the closest-hit shading of RayTracing.rchit (:136-416, NEE :338-350)
@@ -50,6 +56,7 @@ constexpr int kAdjBlock = 128;
 constexpr int kAdjWaves = kAdjBlock / 64;
 constexpr int kSlots = 256;  // LDS table entries per wave
 constexpr int kProbe = 4;    // slots a key tries before its atomics go out directly
+constexpr uint32_t kLightSlots = 256;  // lights summed in LDS (the others: fp64 atomics)
 
 struct AdjView {
     const float4* grad_accum;  // dL/d accum per pixel
@@ -67,10 +74,12 @@ struct WaveTable {
     unsigned long long* keys;
     float4* vals;
     uint32_t* used;
+    double* lights;  // sums of the first kLightSlots lights
     uint32_t lane;
 
     // every lane of the wave
     __device__ void clear() {
+        for (uint32_t s = lane; s < kLightSlots; s += 64) lights[s] = 0.0;
         for (int s = int(lane); s < kSlots; s += 64) {
             keys[s] = 0ull;
             vals[s] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -94,6 +103,23 @@ struct WaveTable {
             }
         }
         return false;
+    }
+    // any lane: `sums` are the frame's
+    __device__ void add_light(double* sums, uint32_t light, double v) {
+        if (v == 0.0) return;
+        if (light < kLightSlots) atomicAdd(&lights[light], v);
+        else atomicAdd(&sums[light], v);
+    }
+    // every lane of the wave: one fp64 atomic per non-zero sum
+    __device__ uint32_t drain_lights(double* sums) {
+        __threadfence_block();
+        uint32_t n = 0;
+        for (uint32_t s = lane; s < kLightSlots; s += 64) {
+            if (lights[s] == 0.0) continue;
+            atomicAdd(&sums[s], lights[s]);
+            n++;
+        }
+        return n;
     }
     __device__ uint32_t occupancy() {
         __threadfence_block();
@@ -193,7 +219,8 @@ struct ReplayTap {
             const rt_light& l = sv.plights[ss.light_index];
             const double v = (gT.x * f.x * double(l.color[0]) + gT.y * f.y * double(l.color[1]) +
                               gT.z * f.z * double(l.color[2])) * ss.light_w;
-            scatter(*tab, true, *gc, av->out.grad_plight + ss.light_index, v, 0.0, 0.0);
+            gc->taps++;
+            tab->add_light(av->out.light_sums, ss.light_index, v);
         }
         const rt_material_raw& mat = *ss.mat;
         if (mat.workflow == RT_WORKFLOW_SPECULAR_GLOSSINESS) return;
@@ -272,7 +299,8 @@ __device__ inline void miss_light_grads(const SceneView& sv, const AdjView& av, 
         const double c = ddot(dnormalize(ld3(li.transform)), rd);
         if (c >= 0.0) continue;
         const double v = -c * k * (gT.x * double(li.color[0]) + gT.y * double(li.color[1]) + gT.z * double(li.color[2]));
-        scatter(tab, true, gc, av.out.grad_dlight + i, v, 0.0, 0.0);
+        gc.taps++;
+        tab.add_light(av.out.light_sums, sv.num_plights + i, v);
     }
 }
 
@@ -281,7 +309,7 @@ __device__ inline void miss_light_grads(const SceneView& sv, const AdjView& av, 
 // on `next_pixel` for the lanes that need one; pixels numbered 8x8 tile by tile, so
 // the lanes a wave serves together sit in one or two tiles).  A wave no longer
 // lasts as long as its slowest pixel.  Each pixel's samples stay in order in one
-// lane, so the gradients are the same up to the order of the float sums.
+// lane, so the gradients are the same up to the order of their sums.
 // Bound by latency at one wave per SIMD, which leaves most of the LDS free: the hits that
 // pass 1 finds at a lane's first kKeptHits bounces stay there for pass 2, which traces
 // again only beyond them (512x512, 16 samples, depth 4: 19.3 ms with every ray traced
@@ -293,11 +321,12 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjoint(FrameArgs fa, AdjView av,
     __shared__ unsigned long long s_keys[kAdjWaves][kSlots];
     __shared__ float4 s_vals[kAdjWaves][kSlots];
     __shared__ uint32_t s_used[kAdjWaves];
+    __shared__ double s_lights[kAdjWaves][kLightSlots];
     __shared__ uint32_t s_hits[kStats ? 1 : kKeptHits * kHitWords * kAdjBlock];
     const uint32_t tiles_x = (fa.width + 7) / 8;
     const uint32_t npix = tiles_x * ((fa.height + 7) / 8) * 64u;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    WaveTable tab{s_keys[wave], s_vals[wave], &s_used[wave], lane};
+    WaveTable tab{s_keys[wave], s_vals[wave], &s_used[wave], s_lights[wave], lane};
     tab.clear();
     PathCounters pc;
     GradCounts gc;
@@ -417,6 +446,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjoint(FrameArgs fa, AdjView av,
         if (tab.occupancy() > uint32_t(kSlots / 2)) gc.atomics += tab.drain();
     }
     gc.atomics += tab.drain();
+    if (av.out.light_sums) gc.atomics += tab.drain_lights(av.out.light_sums);
     if (kStats) {
         flush_counters(fa.counters, pc);
         const unsigned long long t = wave_sum<unsigned long long>(gc.taps);
@@ -425,6 +455,21 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjoint(FrameArgs fa, AdjView av,
             if (t) atomicAdd(&fa.counters[kCntGradTaps], t);
             if (a) atomicAdd(&fa.counters[kCntGradAtomics], a);
         }
+    }
+}
+
+// clears the pixel counter and the light sums
+__global__ __launch_bounds__(256) void k_adjoint_begin(uint32_t* next_pixel, double* sums, uint32_t n) {
+    if (threadIdx.x == 0) *next_pixel = 0u;
+    for (uint32_t i = threadIdx.x; i < n; i += 256) sums[i] = 0.0;
+}
+
+// adds the light sums to the caller's gradients (point lights, then directional ones)
+__global__ __launch_bounds__(256) void k_light_grads(AdjointOut out, uint32_t num_plights, uint32_t n) {
+    for (uint32_t i = threadIdx.x; i < n; i += 256) {
+        const bool point = i < num_plights;
+        float* const g = point ? out.grad_plight : out.grad_dlight;
+        if (g && out.light_sums[i] != 0.0) g[point ? i : i - num_plights] += float(out.light_sums[i]);
     }
 }
 
@@ -443,8 +488,8 @@ int launch_adjoint(const FrameArgs& fa, const float* grad_accum, const AdjointOu
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, kAdjBlock, 0) != hipSuccess || per_cu < 1) per_cu = 1;
     // resident workgroups, no more than it takes to start every 8x8 tile at once
     const uint32_t g = std::min(uint32_t(cus) * uint32_t(per_cu), (tiles + kAdjWaves - 1) / kAdjWaves);
-    hipError_t e = hipMemsetAsync(next_pixel, 0, sizeof(uint32_t), st);
-    if (e != hipSuccess) return int(e);
+    const uint32_t lights = out.light_sums ? fa.sv.num_plights + fa.sv.num_dlights : 0u;
+    hipLaunchKernelGGL(k_adjoint_begin, dim3(1), dim3(256), 0, st, next_pixel, out.light_sums, lights);
     if (stats) {
         if (any_hit) hipLaunchKernelGGL((k_adjoint<true, true>), dim3(g), dim3(kAdjBlock), 0, st, fa, av, next_pixel);
         else hipLaunchKernelGGL((k_adjoint<false, true>), dim3(g), dim3(kAdjBlock), 0, st, fa, av, next_pixel);
@@ -452,6 +497,7 @@ int launch_adjoint(const FrameArgs& fa, const float* grad_accum, const AdjointOu
         if (any_hit) hipLaunchKernelGGL((k_adjoint<true, false>), dim3(g), dim3(kAdjBlock), 0, st, fa, av, next_pixel);
         else hipLaunchKernelGGL((k_adjoint<false, false>), dim3(g), dim3(kAdjBlock), 0, st, fa, av, next_pixel);
     }
+    if (lights) hipLaunchKernelGGL(k_light_grads, dim3(1), dim3(256), 0, st, out, fa.sv.num_plights, lights);
     return int(hipGetLastError());
 }
 

@@ -118,6 +118,8 @@ struct rt_ctx {
     WavefrontState* wavefront = nullptr;
     bool flatten = true;  // RT_OPTION_FLATTEN_IDENTITY_INSTANCES
     float** d_grad_ptrs = nullptr;  // adjoint: device copy of the gradient pointers
+    double* d_light_sums = nullptr;  // adjoint: the frame's sums per light
+    uint64_t light_cap = 0;
     rt_texture* d_batch_tex = nullptr;  // batch: texture descriptors of every item, end to end
     size_t batch_tex_cap = 0;
     uint32_t grad_cap = 0;
@@ -377,6 +379,7 @@ void rt_destroy(rt_ctx* ctx) {
     if (ctx->d_counters) (void)hipFree(ctx->d_counters);
     if (ctx->d_srgb) (void)hipFree(ctx->d_srgb);
     if (ctx->d_grad_ptrs) (void)hipFree(ctx->d_grad_ptrs);
+    if (ctx->d_light_sums) (void)hipFree(ctx->d_light_sums);
     if (ctx->d_batch_tex) (void)hipFree(ctx->d_batch_tex);
     if (ctx->d_err) (void)hipFree(ctx->d_err);
     if (ctx->d_next_pixel) (void)hipFree(ctx->d_next_pixel);
@@ -1040,6 +1043,16 @@ int rt_trace_rays_adjoint(rt_ctx* ctx, rt_tlas tlas, const rt_bindings* b, const
         RT_HIP(ctx, hipMemcpy(ctx->d_grad_ptrs, grad_textures, sizeof(float*) * nt, hipMemcpyHostToDevice),
                "copy gradient pointers");
     }
+    float* const gp = b->num_plights ? d_grad_point_intensity : nullptr;
+    float* const gd = b->num_dlights ? d_grad_directional_intensity : nullptr;
+    const uint64_t lights = gp || gd ? uint64_t(b->num_plights) + b->num_dlights : 0u;
+    if (lights > ctx->light_cap) {
+        if (ctx->d_light_sums) (void)hipFree(ctx->d_light_sums);  // waits for earlier calls
+        ctx->d_light_sums = nullptr;
+        ctx->light_cap = 0;
+        RT_HIP(ctx, hipMalloc(&ctx->d_light_sums, sizeof(double) * lights), "hipMalloc");
+        ctx->light_cap = lights;
+    }
     float** d_ptrs = ctx->d_grad_ptrs;
     FrameArgs fa;
     make_frame(ctx, it->second, b, nullptr, width, height, &fa);
@@ -1047,8 +1060,7 @@ int rt_trace_rays_adjoint(rt_ctx* ctx, rt_tlas tlas, const rt_bindings* b, const
         RT_HIP(ctx, hipMemsetAsync(ctx->d_counters, 0, sizeof(unsigned long long) * kNumCounters, st), "memset");
         RT_HIP(ctx, hipEventRecord(ctx->ev0, st), "hipEventRecord");
     }
-    AdjointOut out{d_ptrs, nt, b->num_plights ? d_grad_point_intensity : nullptr,
-                   b->num_dlights ? d_grad_directional_intensity : nullptr};
+    AdjointOut out{d_ptrs, nt, gp, gd, lights ? ctx->d_light_sums : nullptr};
     rc = launch_adjoint(fa, d_grad_accum, out, kAdjointTableBounces, st, !fa.fully_opaque, stats != nullptr,
                         ctx->d_next_pixel);
     if (rc) return hip_fail(ctx, hipError_t(rc), "adjoint launch");
