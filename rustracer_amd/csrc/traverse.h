@@ -97,12 +97,16 @@ struct TravRay {
     float3 o, inv;
 };
 
-// 1/x of a ray direction, finite: a component of magnitude under 1e-30 counts as
-// +-1e-30.  Over the lengths rays have it moves the ray by less than any padding, and
-// the box test's products stay finite, so an axis-parallel ray is still culled on the
-// axes it does not move along.
-__device__ inline float safe_inv(float x) {
-    return 1.0f / (fabsf(x) < 1e-30f ? copysignf(1e-30f, x) : x);
+// 1/x of the components of a ray direction.  A component of magnitude under 1e-30 of the
+// largest (of 1, for directions longer than that) counts as that magnitude: over the
+// lengths rays have it moves the ray by less than any padding, and the box test's
+// products stay finite, so an axis-parallel ray is still culled on the axes it does not
+// move along.  Directions come in any length; those so short that the products overflow
+// give NaN there, which the box test's minima and maxima pass over: they are not culled.
+__device__ inline float safe_inv(float x, float least) { return 1.0f / (fabsf(x) < least ? copysignf(least, x) : x); }
+__device__ inline float3 safe_inv(float3 d) {
+    const float least = 1e-30f * fminf(fmaxf(fabsf(d.x), fmaxf(fabsf(d.y), fabsf(d.z))), 1.0f);
+    return mk3(safe_inv(d.x, least), safe_inv(d.y, least), safe_inv(d.z, least));
 }
 
 // What one traversal step reads: the 64 bytes of a node, the 48 of a triangle record
@@ -213,7 +217,7 @@ struct Traversal {
             lost = true;
         }
     }
-    __device__ void to_world() { cur = TravRay{o, mk3(safe_inv(d.x), safe_inv(d.y), safe_inv(d.z))}; }
+    __device__ void to_world() { cur = TravRay{o, safe_inv(d)}; }
     __device__ uint32_t enter(const TlasView& tl, uint32_t* stack, uint32_t stride) {
         to_world();
         if (tl.flat_nodes) {
@@ -319,7 +323,7 @@ struct Traversal {
                                 float(m[4] * Dd.x + m[5] * Dd.y + m[6] * Dd.z),
                                 float(m[8] * Dd.x + m[9] * Dd.y + m[10] * Dd.z));
                 cur.o = oo;
-                cur.inv = mk3(safe_inv(od.x), safe_inv(od.y), safe_inv(od.z));
+                cur.inv = safe_inv(od);
                 wr = woop_setup(od);
                 nodes = reinterpret_cast<const QNode*>(pair_u64(w6.x, w6.y));
                 tris = reinterpret_cast<const float4*>(pair_u64(w6.z, w6.w));
