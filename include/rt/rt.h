@@ -15,6 +15,8 @@
  *    is library-owned, behind rt_blas / rt_tlas handles freed explicitly (the
  *    reference frees acceleration structures in Drop, crates/libs/vulkan/src/
  *    ray_tracing/acceleration_structure.rs:270-277).
+ *    A context keeps up to 64 MiB of device scratch between builds and refits (until
+ *    rt_destroy); what a call needs beyond that it allocates and frees itself.
  *  - One context per host thread.  Calls enqueue work on the context's HIP stream
  *    and return; rt_sync() gives the fence semantics the reference gets from
  *    fence.wait (crates/libs/asset_loader/src/acceleration_structures.rs:237-243).
