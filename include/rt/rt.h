@@ -310,9 +310,13 @@ enum {
      * each of them to the end of its pixel's samples in one lane of one launch
      * (the megakernel's loop from the path's state, traversals stepped as in the
      * persistent megakernel) instead of further queue iterations, whose launches
-     * would last as long as their slowest ray while most of the GPU idles.
-     * 0: never.  Same images.  Ignored while
-     * RT_OPTION_STAGE_TIMING is on.  Default 65536. */
+     * would last as long as their slowest ray while most of the GPU idles.  A slot
+     * set that starts with fewer paths than this (one per pixel) runs in that launch
+     * from the start if all sets' paths are also no more than two rounds of the
+     * lanes the launch can hold (131,072 paths on an MI355X), one round where hits
+     * are alpha-tested; RT_OPTION_TRAVERSAL_VARIANT, the refill thresholds and
+     * RT_OPTION_GRAPH then have no effect on the frame.  0: never.  Same images.
+     * Ignored while RT_OPTION_STAGE_TIMING is on.  Default 65536. */
     RT_OPTION_WAVEFRONT_FINISH = 9,
     /* Most triangles per BVH leaf (1 .. 16) of BLASes and flattened BVHs built
      * afterwards: a subtree with at most this many triangles becomes one leaf.
@@ -359,7 +363,9 @@ int rt_set_option(rt_ctx* ctx, uint32_t option, uint64_t value);
  * more than 3 %), and a setting
  * replaces the one it is compared with only when it is more than 1.5 % faster.
  * A variant whose stack ring gives up on a ray of this frame (restart budget) is
- * not a candidate.  Fills *out (may be NULL).  Synchronises the stream. */
+ * not a candidate.  Where the frame runs in the finishing launch alone
+ * (RT_OPTION_WAVEFRONT_FINISH), the refill threshold, variant and graph replay are
+ * left as they are.  Fills *out (may be NULL).  Synchronises the stream. */
 typedef struct rt_tuning {
     uint32_t traversal_variant;
     uint32_t graph;

@@ -1143,11 +1143,21 @@ int rt_autotune(rt_ctx* ctx, rt_tlas tlas, const rt_bindings* b, uint32_t width,
     double best = -1.0;
     auto consider = [&](double ms) { return ms >= 0.0 && (best < 0.0 || ms < best * (1.0 - kAutotuneMargin)); };
     ctx->use_graph = false;
+    // whether the frame runs no queue kernel with these slot sets and this threshold: then
+    // the settings of the queue kernels stay as they are, since probes of them would all
+    // time the same work and choose by its noise
+    auto no_queue = [&](int streams, uint32_t finish) {
+        wavefront_set_streams(ctx->wavefront, streams);
+        wavefront_set_finish(ctx->wavefront, finish);
+        return u.number_of_samples && u.number_of_bounces &&
+               wavefront_runs_no_queue(ctx->wavefront, width, height, !u.fully_opaque, u.debug == 1u);
+    };
     // 1. refill threshold of the traversal kernel (the default variant; the other
     //    settings are tuned under the refill chosen here), against the frame of the
     //    settings the context has
     rc = probe(best);
-    if (rc == RT_OK) {
+    bool inert = rc == RT_OK && best >= 0.0 && no_queue(ctx->streams, ctx->finish);
+    if (rc == RT_OK && !inert) {
         const uint32_t refills[] = {1u, 16u, 32u, 48u, 64u};
         uint32_t chosen = ctx->refill_ext;
         for (uint32_t r : refills) {
@@ -1164,7 +1174,7 @@ int rt_autotune(rt_ctx* ctx, rt_tlas tlas, const rt_bindings* b, uint32_t width,
     //    completed
     const int incumbent = ctx->variant;
     int best_v = best >= 0.0 ? incumbent : -1;
-    for (int v = 0; v < wavefront_num_variants() && rc == RT_OK; v++) {
+    for (int v = 0; v < wavefront_num_variants() && rc == RT_OK && !inert; v++) {
         if (v == incumbent && best_v >= 0) continue;
         ctx->variant = v;
         double ms = -1.0;
@@ -1188,8 +1198,13 @@ int rt_autotune(rt_ctx* ctx, rt_tlas tlas, const rt_bindings* b, uint32_t width,
         uint32_t grid_f = keep_f;
         double grid_ms = -1.0;
         for (int n = 1; n <= wavefront_max_streams() && rc == RT_OK; n++) {
+            bool timed = n == keep_n && inert;  // every threshold that runs no queue is one setting
             for (uint32_t f : finish) {
                 if (n == keep_n && f == keep_f) continue;
+                if (no_queue(n, f)) {
+                    if (timed) continue;
+                    timed = true;
+                }
                 ctx->streams = n;
                 ctx->finish = f;
                 double ms = -1.0;
@@ -1207,8 +1222,10 @@ int rt_autotune(rt_ctx* ctx, rt_tlas tlas, const rt_bindings* b, uint32_t width,
             ctx->finish = keep_f;
         }
     }
+    inert = rc == RT_OK && best >= 0.0 && no_queue(ctx->streams, ctx->finish);
+    if (inert) ctx->use_graph = keep_graph;
     // 5. graph replay
-    if (rc == RT_OK) {
+    if (rc == RT_OK && !inert) {
         ctx->use_graph = true;
         double ms = -1.0;
         rc = probe(ms);
@@ -1219,7 +1236,7 @@ int rt_autotune(rt_ctx* ctx, rt_tlas tlas, const rt_bindings* b, uint32_t width,
     }
     // 6. the traversal variants again, under the settings chosen after them (the
     //    slot sets change how many rays each trace launch holds)
-    if (rc == RT_OK) {
+    if (rc == RT_OK && !inert) {
         int chosen = ctx->variant;
         for (int v = 0; v < wavefront_num_variants() && rc == RT_OK; v++) {
             if (v == chosen) continue;

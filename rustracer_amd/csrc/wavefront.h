@@ -32,6 +32,9 @@ int wavefront_max_streams();
 // Live-path count below which the rest of a slot set's paths are run to completion by
 // one launch of megakernel-style threads (0: never).  Same images.
 void wavefront_set_finish(WavefrontState* s, uint32_t live_paths);
+// Whether a frame of this size starts in that launch under the present settings: then no
+// queue kernel runs, and variant, refill and graph replay have no effect on it.
+bool wavefront_runs_no_queue(WavefrontState* s, uint32_t width, uint32_t height, bool any_hit, bool stats);
 // Renders `count` frames (host array) in one set of queue kernels: their slots are
 // laid end to end and every kernel serves all of them.  Each frame's image is
 // the one launch_wavefront gives it alone.  Frames with no samples or bounces

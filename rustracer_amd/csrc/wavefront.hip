@@ -693,6 +693,27 @@ void enqueue_iteration(const SlotSet<Frames>& set, uint64_t k, hipStream_t s, ty
     mark(1);
 }
 
+// A set that starts with few paths ends in the finishing launch at once, without the two
+// chunks of iterations that pass before its count is known (256x256 pixels, 4 samples:
+// 2.96 ms with them, 1.87 without; 72x72, 1 sample 1.65 and 0.40).  The line is at two
+// rounds of the chip's lanes for all the sets' paths (360x360 pixels of an opaque scene,
+// 32 samples, 1.98 rounds: 34 ms in iterations, 24 in one launch), and at one round
+// where hits are tested for alpha: rays through many instances vary most (360x360: 88 ms
+// in iterations, 102 in one launch; 256x256: 28.5 and 25.5).
+bool starts_in_finish(WavefrontState* ws, const void* k_finish, uint32_t nslots, uint32_t nsets, bool any_hit) {
+    const uint64_t round = uint64_t(ws->grid_for(k_finish, kFinishBlock)) * kFinishBlock;
+    return nslots < ws->finish_below && uint64_t(nslots) * nsets <= (any_hit ? round : 2 * round);
+}
+
+// The CUs of the current device, read once.
+void ensure_cus(WavefrontState* ws) {
+    if (ws->cus != 0) return;
+    int dev = 0, cus = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    ws->cus = std::max(cus, 1);
+}
+
 // The queue loop.  Each slot set runs init, then chunks of kCheckEvery iterations
 // (extend, shade, shadow, resolve) on its own stream, so one set's kernels fill the
 // CUs another set's kernel tails leave idle; every set's stream waits for `st` at
@@ -702,12 +723,7 @@ void enqueue_iteration(const SlotSet<Frames>& set, uint64_t k, hipStream_t s, ty
 template <class Frames>
 int run_wavefront(WavefrontState* ws, const std::vector<SlotSet<Frames>>& sets, uint64_t max_steps, hipStream_t st,
                   bool any_hit, bool stats, int variant, StageTimer* tm, std::string* err) {
-    if (ws->cus == 0) {
-        int dev = 0, cus = 0;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        ws->cus = std::max(cus, 1);
-    }
+    ensure_cus(ws);
     const int nsets = int(sets.size());
     int rc = ensure_streams(ws, nsets, err);
     if (rc) return rc;
@@ -729,18 +745,9 @@ int run_wavefront(WavefrontState* ws, const std::vector<SlotSet<Frames>>& sets, 
         });
     };
     const typename K::FinishFn k_finish = K::finish(any_hit, stats);
-    // A set that starts with few paths ends in the finishing launch at once, without the two
-    // chunks of iterations that pass before its count is known (256x256 pixels, 4 samples:
-    // 2.96 ms with them, 1.87 without; 72x72, 1 sample 1.65 and 0.40).  The line is at two
-    // rounds of the chip's lanes for all the sets' paths (360x360 pixels of an opaque scene,
-    // 32 samples, 1.98 rounds: 34 ms in iterations, 24 in one launch), and at one round
-    // where hits are tested for alpha: rays through many instances vary most (360x360: 88 ms
-    // in iterations, 102 in one launch; 256x256: 28.5 and 25.5).
-    const uint64_t round = uint64_t(ws->grid_for((const void*)k_finish, kFinishBlock)) * kFinishBlock;
-    const uint64_t direct = any_hit ? round : 2 * round;
     bool alive[kMaxStreams], any_alive = false;
     for (int g = 0; g < kMaxStreams; g++)
-        alive[g] = g < nsets && (tm || sets[g].nslots >= ws->finish_below || uint64_t(sets[g].nslots) * nsets > direct);
+        alive[g] = g < nsets && (tm || !starts_in_finish(ws, (const void*)k_finish, sets[g].nslots, uint32_t(nsets), any_hit));
     static_assert(kCheckEvery % 2 == 0, "a chunk ends on queue 0");
     const bool graph = ws->use_graph && !tm;
     if (graph) {
@@ -891,9 +898,19 @@ int run_wavefront(WavefrontState* ws, const std::vector<SlotSet<Frames>>& sets, 
     return rc;
 }
 
-uint32_t frame_tiles(const FrameArgs& fa) { return ((fa.width + 7) / 8) * ((fa.height + 7) / 8); }
+uint32_t frame_tiles(uint32_t width, uint32_t height) { return ((width + 7) / 8) * ((height + 7) / 8); }
+uint32_t frame_tiles(const FrameArgs& fa) { return frame_tiles(fa.width, fa.height); }
 
 }  // namespace
+
+bool wavefront_runs_no_queue(WavefrontState* ws, uint32_t width, uint32_t height, bool any_hit, bool stats) {
+    ensure_cus(ws);
+    const uint32_t tiles = frame_tiles(width, height);
+    const uint32_t nsets = std::max(std::min(uint32_t(ws->streams), tiles), 1u);
+    // (set 0 is the largest)
+    return starts_in_finish(ws, (const void*)Kernels<OneFrame>::finish(any_hit, stats), ((tiles + nsets - 1) / nsets) * 64u,
+                            nsets, any_hit);
+}
 
 int launch_wavefront(WavefrontState* ws, const FrameArgs& fa, hipStream_t st, bool any_hit, bool stats, int variant,
                      StageTimer* tm, std::string* err) {

@@ -180,3 +180,21 @@ def test_both_sides_of_the_direct_start(gpu_ctx, alpha):
         for streams in (1, 2):
             gpu_ctx.set_option(rt.OPTION_WAVEFRONT_STREAMS, streams)
             assert torch.equal(_trace(gpu_ctx, ds, rt.MODE_WAVEFRONT)[0], want), (width, height, streams)
+
+
+@pytest.mark.parametrize("width,height,inert", [(96, 96, True), (BIG, BIG, False)])
+def test_autotune_leaves_settings_without_effect_alone(gpu_ctx, width, height, inert):
+    """A frame that runs no queue kernel says nothing about their settings: the tuner
+    keeps the ones the context has (graph replay on, a variant and a refill threshold
+    other than the defaults), and the image stays the same."""
+    ds = G.device_scene(gpu_ctx, f"queue_tune_{width}", lambda: _cornell(width, height, 2))
+    want, _ = _trace(gpu_ctx, ds, rt.MODE_MEGAKERNEL)
+    gpu_ctx.set_option(rt.OPTION_GRAPH, 1)
+    gpu_ctx.set_option(rt.OPTION_TRAVERSAL_VARIANT, 1)
+    gpu_ctx.set_option(rt.OPTION_EXTEND_REFILL, 40)
+    t = gpu_ctx.autotune(ds.tlas, ds.buffers, ds.scene.ubo, width, height)
+    print(t)
+    if inert:
+        assert t["wavefront_finish"] > 0
+        assert (t["graph"], t["traversal_variant"], t["extend_refill"]) == (1, 1, 40)
+    assert torch.equal(_trace(gpu_ctx, ds, rt.MODE_WAVEFRONT)[0], want)
