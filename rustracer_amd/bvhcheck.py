@@ -2,8 +2,9 @@
 
 A BLAS is valid when, walking from its root: every child reference is in range,
 no node is reached twice, every triangle record of the BLAS lies in exactly one
-leaf, and every triangle lies inside every box on its path from the root, as the
-traversal decodes the quantised boxes (in fp32, no tolerance)."""
+leaf, every child's stack entry is that of its count, and every triangle lies inside
+every box on its path from the root, with the planes that the traversal tests (the
+quantised planes, unrounded; no tolerance)."""
 import numpy as np
 
 from . import rt
@@ -27,7 +28,7 @@ def check_blases(ctx, blases, expect_prims=None):
     out = [None] * len(blases)
     for members in pools.values():
         info0 = infos[members[0]]
-        pool = _Pool(rt.read_nodes(ctx, info0))
+        pool = _Pool(rt.read_qnodes(ctx, info0))
         n_total = max(infos[k].first_prim + infos[k].num_prims for k in members)
         tris = np.frombuffer(rt.read_device(info0.tris, 48 * max(1, n_total)), TRI)[:n_total] if n_total else np.zeros(0, TRI)
         for k in members:
@@ -38,20 +39,30 @@ def check_blases(ctx, blases, expect_prims=None):
 
 
 class _Pool:
-    """The decoded nodes of one node pool, and the per-node scratch of a walk (visit
-    counts, path boxes), which each walk resets on the nodes it reached so that the
-    BLASes of one pool are walked without re-decoding or re-allocating the pool."""
+    """The nodes of one node pool (quantised, or decoded fp32 boxes), and the per-node
+    scratch of a walk (visit counts, path boxes), which each walk resets on the nodes it
+    reached so that the BLASes of one pool are walked without re-decoding or
+    re-allocating the pool."""
 
     def __init__(self, nodes):
         self.n = n = len(nodes)
         self.child = nodes["child"].astype(np.int64)
         self.count = nodes["count"].astype(np.int64)
-        self.lo = np.stack([nodes["lo_x"], nodes["lo_y"], nodes["lo_z"]], -1)  # (n, 4, 3)
-        self.hi = np.stack([nodes["hi_x"], nodes["hi_y"], nodes["hi_z"]], -1)
+        self.entry = np.ones((n, 4), bool)  # whether the child's stack entry is right
+        if nodes.dtype == rt.QNODE:
+            step = np.ldexp(1.0, nodes["exp"].astype(np.int64))[:, :, None]
+            q = nodes["q"].reshape(n, 3, 2, 4).astype(np.float64)
+            origin = nodes["origin"].astype(np.float64)[:, :, None]
+            self.lo = np.swapaxes(origin + q[:, :, 0] * step, 1, 2)  # (n, 4, 3)
+            self.hi = np.swapaxes(origin + q[:, :, 1] * step, 1, 2)
+            self.entry = nodes["tag"] == np.where(self.count > 0, 0x80 | (self.count - 1) << 3, 0)
+        else:
+            self.lo = np.stack([nodes["lo_x"], nodes["lo_y"], nodes["lo_z"]], -1)
+            self.hi = np.stack([nodes["hi_x"], nodes["hi_y"], nodes["hi_z"]], -1)
         self.visits = np.zeros(n, np.int64)
-        # intersection of the decoded boxes on the path to each reached node
-        self.path_lo = np.full((n, 3), -np.inf, np.float32)
-        self.path_hi = np.full((n, 3), np.inf, np.float32)
+        # intersection of the boxes on the path to each reached node
+        self.path_lo = np.full((n, 3), -np.inf, self.lo.dtype)
+        self.path_hi = np.full((n, 3), np.inf, self.lo.dtype)
 
     def reset(self, reached):
         self.visits[reached] = 0
@@ -83,6 +94,8 @@ def _walk(pool, root, first_prim, num_prims, tris, kind, expect_prims, reached):
         valid = c != EMPTY
         if np.any(valid & np.any(lo[frontier] > hi[frontier], -1)):
             errors.append("a child box is inverted")
+        if np.any(valid & ~pool.entry[frontier]):
+            errors.append("a child's stack entry is not that of its count")
         blo = np.maximum(lo[frontier], path_lo[frontier][:, None, :])
         bhi = np.minimum(hi[frontier], path_hi[frontier][:, None, :])
         internal = valid & (cnt == 0)
@@ -146,7 +159,7 @@ def check_tlas(ctx, tlas, num_instances):
     """The TLAS proper, the instance records, and the flattened BVH over identity
     instances: every instance is reached exactly once, through one or the other."""
     info = tlas.info()
-    nodes = rt.read_nodes(ctx, info)
+    nodes = rt.read_qnodes(ctx, info)
     errs = _check(_Pool(nodes), info.root, 0, info.num_prims, None, "instance")
     inst = np.frombuffer(rt.read_device(info.tris, INST.itemsize * max(1, num_instances)), INST)[:num_instances]
     if num_instances and not np.array_equal(np.sort(inst["instance_id"]), np.arange(num_instances)):
@@ -157,7 +170,7 @@ def check_tlas(ctx, tlas, num_instances):
         if nt != num_instances:
             errs.append(f"TLAS reaches {nt} of {num_instances} instances and there is no flattened BVH")
         return errs
-    fnodes = rt.read_nodes(ctx, fi)
+    fnodes = rt.read_qnodes(ctx, fi)
     ftris = np.frombuffer(rt.read_device(fi.tris, 48 * fi.num_prims), TRI)
     errs += _check(_Pool(fnodes), fi.root, 0, fi.num_prims, ftris, "flat")
     bits = ftris["v1"][:, 3].copy().view("<u4")

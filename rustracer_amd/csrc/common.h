@@ -28,7 +28,7 @@ constexpr int kLeafCountShift = 27;          // leaf entry: bits 27..30 = count 
 constexpr uint32_t kLeafFirstMask = (1u << kLeafCountShift) - 1u;
 constexpr int kMaxLeafPrims = 16;
 
-// The builder's 4-wide node with fp32 child boxes (also the decoded form of QNode).
+// The builder's 4-wide node with fp32 child boxes.
 struct alignas(128) WideNode {
     float lo_x[4], hi_x[4], lo_y[4], hi_y[4], lo_z[4], hi_z[4];
     uint32_t child[4];  // internal: node index; leaf: first record; empty: kEmpty
@@ -37,9 +37,11 @@ struct alignas(128) WideNode {
 static_assert(sizeof(WideNode) == 128, "WideNode is 128 bytes");
 
 // The traversal's node, 64 B: the four child boxes as 8-bit steps on a per-axis
-// power-of-two grid anchored at `origin`; a plane is fmaf(q, 2^exp, origin) in
-// fp32.  The builder rounds every plane outward and checks that exact fp32 decode,
-// so a decoded box always contains the child's fp32 box.
+// power-of-two grid anchored at `origin`; a plane is origin + q 2^exp, unrounded.  The
+// builder rounds every plane outward and checks it as an fp32 number, so a plane may lie
+// inside the child's fp32 box by half an ulp, 2^-24 of its coordinate.  The child's box is
+// padded by 2^-20 of the segment's largest coordinate (k_seg_pad), 16 times that: the
+// planes always enclose what the child holds.
 struct alignas(64) QNode {
     float origin[3];
     int8_t exp[3];

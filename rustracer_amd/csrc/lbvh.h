@@ -1,5 +1,5 @@
 // lbvh.h — batched LBVH builder (Morton codes, LDS radix sort, Karras hierarchy,
-// bottom-up box fit, collapse to 4-wide 128-byte nodes).
+// treelets and boxes bottom-up, collapse to 4-wide 64-byte nodes).
 //
 // It builds the structures the Vulkan driver builds for
 // vkCmdBuildAccelerationStructuresKHR in the reference

@@ -100,8 +100,9 @@ __global__ void k_reorder_tris(const float4* in, const uint32_t* perm, uint32_t 
 }
 
 // One axis of a node: the grid (origin, exponent) and the 8-bit planes of the
-// non-empty children, each rounded outward so that the fp32 decode
-// fmaf(q, 2^e, origin) traversal evaluates lies on or outside the child's plane.
+// non-empty children, each rounded outward so that fmaf(q, 2^e, origin) lies on or
+// outside the child's plane.  Traversal takes the plane unrounded, which is at most half
+// an ulp further in: the padding of the child's plane covers it (QNode).
 __device__ inline void quantize_axis(const float lo[4], const float hi[4], const uint32_t child[4], float& origin,
                                      int8_t& exp, uint8_t qlo[4], uint8_t qhi[4]) {
     float o = INFINITY, top = -INFINITY;

@@ -129,7 +129,8 @@ __device__ inline float qbyte(uint32_t w, int k) { return float((w >> (8 * k)) &
 // says which of an axis' two planes comes first.  With u = 2^-24 the rounded distance is
 // off by at most 3u |b| + 3u |t|, b = (origin - o) inv.  Moving b outward by 5u |b| on
 // both sides and the exit by 16u |t| covers both, so a box that the exact ray touches is
-// never rejected (as the widened exit of Ize 2013 does for decoded planes).
+// never rejected (as the widened exit of Ize 2013 does for decoded planes).  The planes
+// enclose the child unrounded (QNode).
 __device__ inline void node_hits(const StepData& n, const TravRay& r, float tmin, float tmax, float key[4],
                                  uint32_t ent[4]) {
     constexpr float kB = 5.0f / 16777216.0f, kT = 16.0f / 16777216.0f;

@@ -532,17 +532,20 @@ def trace_primary(ctx, tlas, buffers, ubo, width, height):
     return d_hits.cpu().numpy().view(L.HIT)
 
 
-def read_nodes(ctx, info):
-    """Copies a BVH's node array (64-byte quantised nodes) to the host and decodes it
-    into NODE records (fp32 child boxes exactly as traversal decodes them)."""
+def read_qnodes(ctx, info):
+    """Copies a BVH's node array (64-byte quantised nodes) to the host."""
     ctx.sync()
-    raw = np.frombuffer(read_device(info.nodes, QNODE.itemsize * info.num_nodes), QNODE)
-    return decode_nodes(raw)
+    return np.frombuffer(read_device(info.nodes, QNODE.itemsize * info.num_nodes), QNODE)
+
+
+def read_nodes(ctx, info):
+    """The same, decoded into NODE records (fp32 child boxes)."""
+    return decode_nodes(read_qnodes(ctx, info))
 
 
 def decode_nodes(raw):
-    """QNode -> NODE: plane = origin + q * 2^exp in fp32 (q * 2^exp is exact, so the
-    single rounding matches the device's fmaf)."""
+    """QNode -> NODE: plane = origin + q * 2^exp, rounded to fp32 as the builder checks it
+    (q * 2^exp is exact)."""
     out = np.zeros(len(raw), NODE)
     scale = np.ldexp(np.float32(1.0), raw["exp"].astype(np.int32)).astype(np.float32)  # (n, 3)
     q = raw["q"].astype(np.float32).reshape(-1, 6, 4)
@@ -557,7 +560,7 @@ def decode_nodes(raw):
 
 
 QNODE = np.dtype([("origin", "<f4", 3), ("exp", "i1", 3), ("_pad0", "u1"), ("q", "u1", 24), ("child", "<u4", 4),
-                  ("count", "u1", 4), ("_pad1", "<u4")])
+                  ("count", "u1", 4), ("tag", "u1", 4)])
 assert QNODE.itemsize == 64
 
 
