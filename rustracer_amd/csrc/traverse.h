@@ -103,10 +103,12 @@ struct TravRay {
 // products stay finite, so an axis-parallel ray is still culled on the axes it does not
 // move along.  Directions come in any length; those so short that the products overflow
 // give NaN there, which the box test's minima and maxima pass over: they are not culled.
-__device__ inline float safe_inv(float x, float least) { return 1.0f / (fabsf(x) < least ? copysignf(least, x) : x); }
+// (The limit is put on the reciprocals: a division then waits for no comparison.)
 __device__ inline float3 safe_inv(float3 d) {
-    const float least = 1e-30f * fminf(fmaxf(fabsf(d.x), fmaxf(fabsf(d.y), fabsf(d.z))), 1.0f);
-    return mk3(safe_inv(d.x, least), safe_inv(d.y, least), safe_inv(d.z, least));
+    const float3 r = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+    const float most = 1e30f * fmaxf(fminf(fabsf(r.x), fminf(fabsf(r.y), fabsf(r.z))), 1.0f);
+    return mk3(copysignf(fminf(fabsf(r.x), most), r.x), copysignf(fminf(fabsf(r.y), most), r.y),
+               copysignf(fminf(fabsf(r.z), most), r.z));
 }
 
 // What one traversal step reads: the 64 bytes of a node, the 48 of a triangle record
