@@ -464,12 +464,13 @@ __global__ __launch_bounds__(256) void k_adjoint_begin(uint32_t* next_pixel, dou
     for (uint32_t i = threadIdx.x; i < n; i += 256) sums[i] = 0.0;
 }
 
-// adds the light sums to the caller's gradients (point lights, then directional ones)
+// adds the light sums to the caller's gradients (point lights, then directional ones),
+// which another context's call may be adding to
 __global__ __launch_bounds__(256) void k_light_grads(AdjointOut out, uint32_t num_plights, uint32_t n) {
     for (uint32_t i = threadIdx.x; i < n; i += 256) {
         const bool point = i < num_plights;
         float* const g = point ? out.grad_plight : out.grad_dlight;
-        if (g && out.light_sums[i] != 0.0) g[point ? i : i - num_plights] += float(out.light_sums[i]);
+        if (g && out.light_sums[i] != 0.0) atomicAdd(&g[point ? i : i - num_plights], float(out.light_sums[i]));
     }
 }
 

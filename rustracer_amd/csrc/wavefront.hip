@@ -696,10 +696,12 @@ void enqueue_iteration(const SlotSet<Frames>& set, uint64_t k, hipStream_t s, ty
 // A set that starts with few paths ends in the finishing launch at once, without the two
 // chunks of iterations that pass before its count is known (256x256 pixels, 4 samples:
 // 2.96 ms with them, 1.87 without; 72x72, 1 sample 1.65 and 0.40).  The line is at two
-// rounds of the chip's lanes for all the sets' paths (360x360 pixels of an opaque scene,
-// 32 samples, 1.98 rounds: 34 ms in iterations, 24 in one launch), and at one round
-// where hits are tested for alpha: rays through many instances vary most (360x360: 88 ms
-// in iterations, 102 in one launch; 256x256: 28.5 and 25.5).
+// rounds of the chip's lanes for all the sets' paths: up to there the one launch was ahead
+// for a room of 5,000 triangles and a sphere of 2M at 64x64 to 360x360 pixels and 1, 4 and
+// 32 samples, least at 360x360 (1.98 rounds) and 32 (18.7 ms in iterations, 18.3 in one
+// launch; 36.1 and 26.4).  It is at one round where hits are tested for alpha: rays
+// through many instances vary most (1000 instances, 256x256, 4 samples: 18.8 and 17.7 ms;
+// 360x360, which would be two rounds, took longer in one launch).
 bool starts_in_finish(WavefrontState* ws, const void* k_finish, uint32_t nslots, uint32_t nsets, bool any_hit) {
     const uint64_t round = uint64_t(ws->grid_for(k_finish, kFinishBlock)) * kFinishBlock;
     return nslots < ws->finish_below && uint64_t(nslots) * nsets <= (any_hit ? round : 2 * round);
